@@ -296,7 +296,11 @@ typedef struct {
     int slices_per_item; /* LINEAR modes: slices of identical geometry back-projected together, sharing
                           * each pixel's coordinate and LDS reads: 0 (default) = four per work item
                           * with FP32 values in LDS (results identical to one per item; a class's
-                          * leftovers as a pair and a single), sixteen with FP16 pairs (lds_half:
+                          * leftovers as a pair and a single), every 64 slices of one geometry of
+                          * larger FP32 images (from 640^2 pixels, 256 projections and 5e8 updates
+                          * per slice on, tile 0) on the matrix cores instead (each value as
+                          * two FP16 halves, FP32 sums: closer to FP64 than the vector kernels, not bit
+                          * for bit theirs; ask for 4 to have those), sixteen with FP16 pairs (lds_half:
                           * one FP16 dot product per update and one power-of-two scale per work
                           * item; eight on the 64x64 tile, which has no sixteen-slice kernel); or
                           * 1, 2, 4, 8, 16, 32 (at most 4 with FP32 values in LDS; 8 on the 64x64,

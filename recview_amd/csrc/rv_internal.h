@@ -120,21 +120,31 @@ inline int output_irad2(int N, double center, int iInterpolation)
 // (BP_LINEAR4: four);
 // BP_LINEAR_H2 / H4 / H8 / H16: BP_LINEAR_H over two / four / eight / sixteen;
 // BP_LINEAR_M32: 32 FP16 slices per work item, the updates done as matrix
-// products on the MFMA units (the others in BpSlice::rows_x / scales_x / out_x).
+// products on the MFMA units (the others in BpSlice::rows_x / scales_x / out_x);
+// BP_LINEAR_X64: 64 FP32 slices per work item as matrix
+// products of operands split into two FP16 halves.
 enum BpMode {
     BP_LINEAR = 0, BP_LUT_F32 = 1, BP_LUT_I32 = 2, BP_LINEAR_H = 3, BP_LINEAR2 = 4,
     BP_LINEAR_H2 = 5, BP_LINEAR_H4 = 6, BP_LINEAR_H8 = 7, BP_LINEAR_H16 = 8, BP_LINEAR_M32 = 9,
-    BP_LINEAR4 = 10
+    BP_LINEAR4 = 10, BP_LINEAR_X64 = 11
 };
 constexpr int bp_slices_per_item(int mode)
 {
     return (mode == 4 || mode == 5) ? 2 : (mode == 6 || mode == 10) ? 4 : mode == 7 ? 8 : mode == 8 ? 16
-         : mode == 9 ? 32 : 1;
+         : mode == 9 ? 32 : mode == 11 ? 64 : 1;
 }
-constexpr int BP_MAX_SLICES_PER_ITEM = 32;
+constexpr int BP_MAX_SLICES_PER_ITEM = 64;
 // BP_LINEAR_M32 packed rows: per angle row, (N + 7) / 8 chunks of eight samples,
 // each chunk the 32 slices' samples side by side (16 B per slice)
 constexpr long long bp_m32_chunks(int N) { return (N + 7) / 8; }
+// BP_LINEAR_X64 packed rows: per angle row one plane per 16 slices of
+// bpx_pairs(N) sample pairs x 16 slices x (high FP16 halves, low FP16 halves) of the
+// FP32 samples, kBpxPad zero samples before the row and at least as many after it
+constexpr int kBpxPad = 48;
+constexpr int bpx_pairs(int N) { return (N + 1) / 2 + kBpxPad; }
+constexpr int bpx_angles(int nang) { return (nang + 3) / 4 * 4; }
+constexpr int kBpxParts = 64;           // partial maxima per slice
+constexpr int kBpxPart = 64 * 32 * 32;  // sums of one work item (a segment's totals)
 
 // Per-angle table entry.  LINEAR: detector coordinate of pixel (ix, iy) of the
 // output grid is u = u0 + ix*dux + iy*duy (all double).  LUT16: the reference
@@ -168,6 +178,10 @@ struct BpSlice {
     // bits), [tiles][nang], built once per plan, read one angle ahead instead of
     // formed in LDS per chunk; nullptr: formed per chunk
     const float4* tgeom;
+    // BP_LINEAR_X64: filtered rows of the item's first slice (rows_x: the others'), and
+    // [slice][angle] 1 where such a row has a sample that is not finite
+    const void* rows_0;
+    unsigned char* bad;
 };
 
 struct BpLaunch {
@@ -188,6 +202,7 @@ struct BpLaunch {
     int ang_begin, ang_end; // ang_end > 0: only the slice's angles [ang_begin, ang_end)
                             // (a segment of a launch sequence); 0: all of them
     int tgeom;              // BP_LINEAR2: 1 = every slice has BpSlice::tgeom
+    float* part;            // BP_LINEAR_X64: kBpxPart floats per workgroup
 };
 
 // Persistent launches take work-list positions from kXcds counters: the list is
@@ -243,6 +258,7 @@ struct PackJob {
     int nrows, N;           // rows of N samples, row stride N
     void* out;              // [nrows][N] packed samples
     float* gscale;          // FP16 pairs: the item scale, written by the scale pass
+    unsigned char* bad;     // BP_LINEAR_X64: BpSlice::bad, written by the pack pass
 };
 // Item scales of FP16-pair jobs (jobs of other kinds are skipped), then the
 // packing of njobs jobs of one kind (0: FP32 pairs; 3: FP32, four slices; 2 / 4 /
@@ -273,6 +289,14 @@ bool bp_has_tgeom(int mode);                // the mode has a tile geometry tabl
 bool bp_deals_runs(int mode);               // persistent work dealt to the XCDs in runs
 int bp_max_chunk(int mode);                 // largest chunk a mode supports
 size_t bp_lds_bytes(int mode, int tile, int chunk);
+// BP_LINEAR_X64: kernel attributes (outside stream captures), tile geometry table of
+// 32 x 32 tiles ([tiles][bpx_angles(nang)]), packing of njobs jobs of ns slices (part:
+// njobs * BP_MAX_SLICES_PER_ITEM * kBpxParts floats) and back-projection.
+void bpx_prepare();
+void launch_bpx_geometry(const AngleEntry* ang, int nang, int tiles_x, int ntiles, int N, float4* out,
+                         hipStream_t stream);
+void launch_bpx_pack(const PackJob* d_jobs, int njobs, int ns, int max_rows, float* part, hipStream_t stream);
+void launch_bpx(const BpLaunch& L, int grid, hipStream_t stream);
 void launch_zero_u32(unsigned int* p, int n, hipStream_t stream);
 // Tile geometry table of BpSlice::tgeom for tiles of tw x th pixels, ntiles of them
 // in rows of tiles_x, over nang angle entries.

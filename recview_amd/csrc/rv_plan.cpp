@@ -24,6 +24,20 @@
 
 namespace {
 
+constexpr bool is_x(int mode) { return mode == rv::BP_LINEAR_X64; }
+
+// Stacks that run BP_LINEAR_X64 (64 slices per work item on the matrix cores) instead
+// of four slices per item on the vector ALU: the item's 32 x 32 tiles have to fill the
+// 256 CUs more than once, and its prologue and 16-byte image writes have to be few
+// beside the angles.  Measured for 64 slices, whole execution, four per item against
+// 64 per item (ms): 2048^2 x 1800 38.3 / 31.1, 1024^2 x 900 5.07 / 4.38, 700^2 x 700
+// 2.12 / 1.89, 640^2 x 225 0.68 / 0.68, 2048^2 x 60 1.53 / 1.60, 512^2 x 450 0.81 /
+// 0.83; 70 slices of 800^2 x 300 1.49 / 1.63 (the six slices left over run apart).
+bool x64_pays(int out_n, int nang)
+{
+    return out_n >= 640 && nang >= 256 && (double)out_n * out_n * nang >= 5e8;
+}
+
 struct SliceState {
     RvSliceSpec spec;
     std::vector<float> fdeg;     // angles of the reconstructed rows
@@ -45,6 +59,8 @@ struct SliceState {
     size_t stitch_off = 0;       // element offset in the stitch buffer
     size_t pair_off = 0;         // first entry in the pair table
 };
+
+constexpr int kPackX = 100;      // PackRange::kind of BP_LINEAR_X64 jobs: kPackX + slices
 
 struct Group {
     int tile = 0, chunk = 0;
@@ -84,6 +100,8 @@ struct rv_plan_opaque {
     rv::PackJob* d_pack_jobs = nullptr;
     int n_pack = 0;
     bool pack_half = false;
+    float* d_xpart = nullptr;            // BP_LINEAR_X64 packing: partial maxima
+    float* d_xsum = nullptr;             // BP_LINEAR_X64: segment totals, per workgroup
     struct PackRange { int first, count, kind, rows; };
     std::vector<PackRange> pack_ranges;  // one per group: jobs of one kind
     void* d_fft_work = nullptr;          // two-pass transforms (n > 16384): work rows
@@ -122,6 +140,8 @@ void plan_free(rv_plan_t p)
     (void)hipFree(p->d_gscale);
     (void)hipFree(p->d_tgeom);
     (void)hipFree(p->d_pack_jobs);
+    (void)hipFree(p->d_xpart);
+    (void)hipFree(p->d_xsum);
     (void)hipFree(p->d_fft_work);
     delete p;
 }
@@ -277,8 +297,12 @@ int launch_filters(rv_plan_t p, const void* const* d_sino, hipStream_t st)
 void launch_packing(rv_plan_t p, hipStream_t st)
 {
     if (p->pack_half) rv::launch_pack_scales(p->d_pack_jobs, p->n_pack, st);
-    for (const auto& R : p->pack_ranges)
-        rv::launch_pack(p->d_pack_jobs + R.first, R.count, R.kind, p->store, R.rows, st);
+    for (const auto& R : p->pack_ranges) {
+        if (R.kind >= kPackX)
+            rv::launch_bpx_pack(p->d_pack_jobs + R.first, R.count, R.kind - kPackX, R.rows, p->d_xpart, st);
+        else
+            rv::launch_pack(p->d_pack_jobs + R.first, R.count, R.kind, p->store, R.rows, st);
+    }
 }
 
 int launch_backprojection(rv_plan_t p, hipStream_t st, bool pack = true)
@@ -299,6 +323,13 @@ int launch_backprojection(rv_plan_t p, hipStream_t st, bool pack = true)
         L.chunk = G.chunk;
         L.tile = G.tile;
         L.tgeom = G.tgeom ? 1 : 0;
+        if (is_x(G.mode)) {
+            rv::launch_zero_u32(ctr, rv::kXcds * rv::kCounterStride, st);
+            L.counter = ctr;
+            L.part = p->d_xsum;
+            rv::launch_bpx(L, G.grid, st);
+            continue;
+        }
         if (L.counter) rv::launch_zero_u32(ctr, rv::kXcds * rv::kCounterStride, st);
         rv::launch_bp(L, G.grid, st);
     }
@@ -477,9 +508,9 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
         opt->slices_per_item != 4 && opt->slices_per_item != 8 && opt->slices_per_item != 16 &&
         opt->slices_per_item != 32)
         return fail(p, "slices_per_item must be 0, 1, 2, 4, 8, 16 or 32");
-    // default: four FP32 slices or sixteen FP16-pair slices per item, all on the
-    // vector ALU (packed rows; sixteen form on the 32x64 and 32x32 tiles, eight on
-    // 64x64).  Measured per 2048^2 x 1800 slice (64-slice stack): FP32 0.57 ms with
+    // default: sixty-four FP32 slices per item on the matrix cores where x64_pays, else
+    // four FP32 slices or sixteen FP16-pair slices per item on the vector ALU (packed
+    // rows; sixteen form on the 32x64 and 32x32 tiles, eight on 64x64).  Measured per 2048^2 x 1800 slice (64-slice stack): FP32 0.57 ms with
     // four per item, 0.58 ms with two; FP16 pairs 0.367 / 0.381 / 0.492 ms with
     // sixteen (32x64) / eight (64x64) / four per item.  A class's leftovers run as
     // a pair and a single.  32 per item (opt-in) runs the matrix-core kernel: 0.343 ms.
@@ -523,6 +554,14 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
         for (int s = 0; s < nslices; s++) classes.push_back({s});
     }
 
+    // RECVIEW_GEOMETRY_TABLES=0 (diagnostics, tests): every group forms its geometry
+    // per chunk, as when the tables would exceed the budget
+    const char* tg_env = std::getenv("RECVIEW_GEOMETRY_TABLES");
+    const bool tg_allowed = !(tg_env && tg_env[0] == '0');
+    const size_t tg_budget = (size_t)8 << 30;
+    size_t tg_total = 0;
+    std::map<int, std::pair<size_t, int>> xg_tab;                  // class -> (offset, slice) of its X table
+
     // groups by tile configuration and slices per item; work items cost-sorted within each group
     std::map<std::pair<int, int>, int> gidx;
     for (const auto& cls : classes) {
@@ -532,7 +571,25 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
             const int tile = p->sl[cls[i]].tile;
             const bool tile8 = tile == 0 || tile == 2 || tile == 4;    // eight per item: 64^2, 32^2, 32x64
             const bool tile16 = tile == 2 || tile == 4;                // sixteen: 32^2 and 32x64
-            const int k = (per_item >= 32 && left >= 32) ? 32                  // matrix cores, 32x32 tiles
+            // FP32 stacks on the matrix cores (default plans only: an explicit
+            // slices_per_item keeps the vector kernels and their rounding)
+            int kx = 0;
+            if (p->mode == rv::BP_LINEAR && p->store == 0 && opt->slices_per_item == 0 && tg_allowed && left >= 64 &&
+                tile == 0 && x64_pays(p->sl[cls[i]].out_n, p->sl[cls[i]].nang)) {
+                const int c = (int)(&cls - classes.data());
+                const SliceState& S = p->sl[cls[i]];
+                const size_t side = (S.out_n + rv::bp_tile_side(2) - 1) / rv::bp_tile_side(2);
+                const size_t bytes = align_up(side * side * rv::bpx_angles(S.nang) * 16, 256);
+                if (xg_tab.count(c) || tg_total + bytes <= tg_budget) {
+                    if (!xg_tab.count(c)) {
+                        xg_tab[c] = std::make_pair(tg_total, cls[i]);
+                        tg_total += bytes;
+                    }
+                    kx = 64;
+                }
+            }
+            const int k = kx ? kx
+                        : (per_item >= 32 && left >= 32) ? 32                  // matrix cores, 32x32 tiles
                         : (per_item >= 16 && left >= 16 && tile16) ? 16
                         : (per_item >= 8 && left >= 8 && tile8) ? 8
                         : (per_item >= 4 && left >= 4) ? 4 : (per_item >= 2 && left >= 2) ? 2 : 1;
@@ -542,14 +599,15 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
             // (2048^2 x 1800: 37.6 vs 45.9 ms for two per item, 52.7 vs 76.0 ms for
             // one), unless the plan asked for at most two per item
             const bool narrow_fp32 = half && per_item > 2;
-            if (k == 32)
+            if (kx || k == 32)
                 for (int e = 0; e < k; e++) {
                     SliceState& T = p->sl[cls[i + e]];
                     T.tile = 2;
                     T.tiles_x = (T.out_n + rv::bp_tile_side(2) - 1) / rv::bp_tile_side(2);
                     T.tiles_y = (T.out_n + rv::bp_tile_h(2) - 1) / rv::bp_tile_h(2);
                 }
-            const int mode = k == 32 ? (int)rv::BP_LINEAR_M32
+            const int mode = kx ? (int)rv::BP_LINEAR_X64
+                           : k == 32 ? (int)rv::BP_LINEAR_M32
                            : k == 16 ? (int)rv::BP_LINEAR_H16
                            : k == 8 ? (int)rv::BP_LINEAR_H8
                            : k == 4 ? (half ? (int)rv::BP_LINEAR_H4 : (int)rv::BP_LINEAR4)
@@ -562,10 +620,10 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
                 Group G;
                 G.tile = p->sl[s].tile;
                 G.mode = mode;
-                G.chunk = p->sl[s].spec.chunk > 0 ? p->sl[s].spec.chunk
+                G.chunk = kx ? 4 : p->sl[s].spec.chunk > 0 ? p->sl[s].spec.chunk
                         : opt->angles_per_chunk > 0 ? opt->angles_per_chunk : rv::bp_default_chunk(mode, G.tile);
                 if (G.chunk > rv::bp_max_chunk(mode)) G.chunk = rv::bp_max_chunk(mode);
-                while (G.chunk > 1 && rv::bp_lds_bytes(mode, G.tile, G.chunk) > 160 * 1024) G.chunk /= 2;
+                while (!kx && G.chunk > 1 && rv::bp_lds_bytes(mode, G.tile, G.chunk) > 160 * 1024) G.chunk /= 2;
                 p->groups.push_back(G);
             }
             Group& G = p->groups[gidx[gk]];
@@ -603,20 +661,25 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
     // 32 / 64 B per sample (two / four / eight / sixteen slices); 32 FP16 slices in
     // chunks of eight samples
     auto packed_size = [](int mode) -> size_t {
-        return mode == rv::BP_LINEAR_M32 ? 64 : mode == rv::BP_LINEAR_H16 ? 64 : mode == rv::BP_LINEAR_H8 ? 32
+        return is_x(mode) ? 4 * (size_t)rv::bp_slices_per_item(mode)
+             : mode == rv::BP_LINEAR_M32 ? 64 : mode == rv::BP_LINEAR_H16 ? 64 : mode == rv::BP_LINEAR_H8 ? 32
              : mode == rv::BP_LINEAR4 ? 32
              : mode == rv::BP_LINEAR2 || mode == rv::BP_LINEAR_H4 ? 16 : mode == rv::BP_LINEAR_H2 ? 8 : 0;
     };
     auto packed_row = [&](int mode, int N) -> size_t {     // bytes per angle row
+        if (is_x(mode)) return (size_t)rv::bpx_pairs(N) * 64 * 2 * (rv::bp_slices_per_item(mode) / 16);
         return mode == rv::BP_LINEAR_M32 ? (size_t)rv::bp_m32_chunks(N) * 8 * packed_size(mode)
                                          : (size_t)N * packed_size(mode);
     };
+    auto packed_rows = [](int mode, int nang) -> size_t { return is_x(mode) ? rv::bpx_angles(nang) : nang; };
     size_t packed_bytes = 0, n_half = 0;
     for (const auto& G : p->groups)
         if (packed_size(G.mode))
             for (int s : G.slices) {
-                packed_bytes += align_up((size_t)p->sl[s].nang * packed_row(G.mode, p->sl[s].g.N), 256);
-                n_half += G.mode != rv::BP_LINEAR2 && G.mode != rv::BP_LINEAR4;
+                packed_bytes += align_up(packed_rows(G.mode, p->sl[s].nang) * packed_row(G.mode, p->sl[s].g.N), 256);
+                if (is_x(G.mode)) packed_bytes += align_up((size_t)64 * p->sl[s].nang, 256);   // BpSlice::bad
+                n_half += is_x(G.mode) ? (size_t)rv::bp_slices_per_item(G.mode)
+                                              : G.mode != rv::BP_LINEAR2 && G.mode != rv::BP_LINEAR4;
             }
     std::vector<rv::PackJob> pack_jobs;
     if (packed_bytes &&
@@ -637,11 +700,6 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
     for (size_t c = 0; c < classes.size(); c++)
         for (int s : classes[c]) cls_of[s] = (int)c;
     std::map<std::pair<int, int>, std::pair<size_t, int>> tg_tab;   // (class, tile) -> (offset, slice)
-    size_t tg_total = 0;
-    // RECVIEW_GEOMETRY_TABLES=0 (diagnostics, tests): every group forms its geometry
-    // per chunk, as when the tables would exceed the budget
-    const char* tg_env = std::getenv("RECVIEW_GEOMETRY_TABLES");
-    const bool tg_allowed = !(tg_env && tg_env[0] == '0');
     for (auto& G : p->groups) {
         if (!tg_allowed || !rv::bp_has_tgeom(G.mode)) continue;
         G.tgeom = true;
@@ -653,7 +711,7 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
             if (tg_tab.count(key)) continue;
             // + 64 B: a chunk's prefetch may read one entry past the tile's last
             const size_t bytes = align_up((size_t)S.tiles_x * S.tiles_y * S.nang * 16 + 64, 256);
-            if (tg_total + bytes > ((size_t)8 << 30)) { G.tgeom = false; break; }
+            if (tg_total + bytes > tg_budget) { G.tgeom = false; break; }
             tg_tab[key] = std::make_pair(tg_total, s);
             tg_total += bytes;
         }
@@ -670,10 +728,16 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
                                      rv::bp_tile_side(S.tile), rv::bp_tile_h(S.tile),
                                      (float4*)(p->d_tgeom + kv.second.first), nullptr);
         }
+        for (const auto& kv : xg_tab) {
+            const SliceState& S = p->sl[kv.second.second];
+            rv::launch_bpx_geometry(p->d_ang + S.ang_off, S.nang, S.tiles_x, S.tiles_x * S.tiles_y, S.g.N,
+                                    (float4*)(p->d_tgeom + kv.second.first), nullptr);
+        }
         if (!rv::hip_ok(hipGetLastError(), "tile geometry") || !rv::hip_ok(hipDeviceSynchronize(), "tile geometry"))
             return fail(p, std::string("plan set-up failed: ") + RecviewLastMessage());
     }
 
+    int x_grid = 0;
     for (auto& G : p->groups) {
         // slice order inside the group: longest projection lists first
         std::vector<int> ord = G.slices;
@@ -688,6 +752,16 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
         order.reserve(base);
         for (int s : ord) {
             const SliceState& S = p->sl[s];
+            if (is_x(G.mode)) {
+                // blocks of 8 x 4 tiles: the 32 workgroups of one XCD read overlapping
+                // detector segments
+                for (int by = 0; by < S.tiles_y; by += 4)
+                    for (int bx = 0; bx < S.tiles_x; bx += 8)
+                        for (int y = by; y < std::min(by + 4, S.tiles_y); y++)
+                            for (int x = bx; x < std::min(bx + 8, S.tiles_x); x++)
+                                order.push_back(S.tile_base + y * S.tiles_x + x);
+                continue;
+            }
             for (int t = 0; t < S.tiles_x * S.tiles_y; t++) order.push_back(S.tile_base + t);
         }
         G.h.resize(G.slices.size());
@@ -710,7 +784,9 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
             B.lut_formula = opt->lut_formula ? 1 : 0;
             B.store = p->store;
             B.out_scale = opt->normalize ? (float)(6.283185307179586 / S.nang) : 1.f;
-            B.tgeom = G.tgeom ? tg_of(G.slices[q]) : nullptr;
+            B.tgeom = is_x(G.mode)
+                          ? (const float4*)(p->d_tgeom + xg_tab.at(cls_of[G.slices[q]]).first)
+                          : G.tgeom ? tg_of(G.slices[q]) : nullptr;
             for (int e = 0; e + 1 < rv::BP_MAX_SLICES_PER_ITEM; e++) {
                 const int s2 = G.others[q][e];
                 if (s2 < 0) continue;
@@ -730,14 +806,17 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
                 J.ang = B.ang;
                 J.nang = S.nang;
                 J.ns = ns;
-                J.half = G.mode != rv::BP_LINEAR2 && G.mode != rv::BP_LINEAR4;
+                const bool x = is_x(G.mode);
+                J.half = !x && G.mode != rv::BP_LINEAR2 && G.mode != rv::BP_LINEAR4;
                 J.store = p->store;
                 J.nrows = S.nang;
                 J.N = S.g.N;
                 J.out = p->d_packed + packed_off;
-                J.gscale = J.half ? p->d_gscale + half_idx++ : nullptr;
+                J.gscale = J.half || x ? p->d_gscale + half_idx : nullptr;
+                half_idx += J.half ? 1 : x ? ns : 0;
                 if (q == 0)
-                    p->pack_ranges.push_back({(int)pack_jobs.size(), 0, J.half ? ns : ns == 4 ? 3 : 0, 0});
+                    p->pack_ranges.push_back(
+                        {(int)pack_jobs.size(), 0, x ? kPackX + ns : J.half ? ns : ns == 4 ? 3 : 0, 0});
                 auto& R = p->pack_ranges.back();
                 R.count++;
                 R.rows = std::max(R.rows, S.nang);
@@ -746,7 +825,12 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
                 B.rows = J.out;                    // the kernel reads the packed rows
                 B.row_stride = G.mode == rv::BP_LINEAR_M32 ? rv::bp_m32_chunks(S.g.N) : S.g.N;
                 B.gscale = J.gscale;
-                packed_off += align_up((size_t)S.nang * packed_row(G.mode, S.g.N), 256);
+                packed_off += align_up(packed_rows(G.mode, S.nang) * packed_row(G.mode, S.g.N), 256);
+                if (x) {
+                    pack_jobs.back().bad = B.bad = p->d_packed + packed_off;
+                    B.rows_0 = J.rows[0];
+                    packed_off += align_up((size_t)64 * S.nang, 256);
+                }
             }
         }
         if (!rv::hip_ok(hipMalloc(&G.d_slices, sizeof(rv::BpSlice) * G.h.size()), "slice table") ||
@@ -755,6 +839,12 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
             !rv::hip_ok(hipMemcpy(G.d_slices, G.h.data(), sizeof(rv::BpSlice) * G.h.size(), hipMemcpyHostToDevice),
                         "slices"))
             return fail(p, std::string("plan upload failed: ") + RecviewLastMessage());
+        if (is_x(G.mode)) {
+            rv::bpx_prepare();
+            G.grid = std::min(rv::device_cu_count(device), G.total_items);     // one workgroup per CU
+            x_grid = std::max(x_grid, G.grid);
+            continue;
+        }
         (void)rv::bp_blocks_per_cu_tg(G.mode, G.tile, G.chunk, G.tgeom);     // sets LDS attributes outside capture
         if (opt->persistent) {
             const int per_cu = rv::bp_blocks_per_cu_tg(G.mode, G.tile, G.chunk, G.tgeom);
@@ -764,6 +854,15 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
         }
     }
     p->cur_out.assign(nslices, nullptr);
+    if (!xg_tab.empty()) {
+        size_t n = 0;
+        for (const auto& R : p->pack_ranges)
+            if (R.kind >= kPackX) n = std::max(n, (size_t)R.count);
+        if (!rv::hip_ok(hipMalloc(&p->d_xpart, sizeof(float) * n * rv::BP_MAX_SLICES_PER_ITEM * rv::kBpxParts),
+                        "partial maxima") ||
+            !rv::hip_ok(hipMalloc(&p->d_xsum, sizeof(float) * rv::kBpxPart * x_grid), "segment totals"))
+            return fail(p, std::string("plan allocation failed: ") + RecviewLastMessage());
+    }
     if (!pack_jobs.empty()) {
         p->n_pack = (int)pack_jobs.size();
         if (!rv::hip_ok(hipMalloc(&p->d_pack_jobs, sizeof(rv::PackJob) * pack_jobs.size()), "pack jobs") ||

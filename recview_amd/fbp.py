@@ -94,7 +94,9 @@ class FbpPlan:
         operation order (bit-identical filtered rows) instead of two rows per transform.
         slices_per_item: LINEAR modes back-project slices of identical geometry
         together (0: four per work item with FP32 values in LDS -- the same results
-        as one per item; a class's leftovers as a pair and a single -- and with FP16
+        as one per item; a class's leftovers as a pair and a single; every 64 slices of
+        one geometry of larger images on the matrix cores, FP32 values as two FP16
+        halves, to FP32 rounding the same -- and with FP16
         pairs (lds_half) sixteen on the 32x64 and 32x32 tiles, eight on 64x64; or 1,
         2, 4, 8, 16, 32, where 8 and up need FP16 pairs, 16 the 32x32 or 32x64
         tile, and 32 selects the matrix-core

@@ -715,3 +715,60 @@ def test_plan_geometry_tables_equal_per_chunk_geometry(monkeypatch):
         _, tables = _run(specs, sinos, **kw)
         for i in range(len(specs)):
             assert np.array_equal(per_chunk[i], tables[i]), (tile, persistent, spi, i)
+
+
+@pytest.mark.parametrize("W,P,S,kw,persistent", [
+    (640, 1221, 64, {}, True),                                         # smallest side; angles 4 k + 1
+    (701, 1018, 65, {}, False),                                        # odd side, a slice left over, angles 4 k + 2
+    (1024, 479, 64, dict(center=490.25), True),                        # axis off the middle: tiles past both row ends
+    (640, 512, 129, dict(out_n=1000, pix_zoom=2.0, x0=-60.5, y0=300.0), False)])   # region partly off the detector
+def test_plan_stack_on_matrix_cores(W, P, S, kw, persistent):
+    """64 FP32 slices of one geometry per work item on the matrix cores (default plans of
+    larger images) against one slice per item and against the FP64 oracle: within FP32
+    rounding everywhere (2e-6 of the range RMS as every FP32 mode; 2e-5 of the range
+    at any pixel: 1/8 of an FP32 step per projection, summed over at most 1221), row ends
+    included, and no further from FP64 than one slice per item."""
+    base, fdeg, c = _sino(W, P, 2600 + W, photons=1e4)
+    center = kw.pop("center", c)
+    gen = torch.Generator().manual_seed(W)
+    gain = torch.rand(S, 1, 1, generator=gen) + 0.25
+    sinos = [(torch.from_numpy(base) * gain[i]).roll(i % 7, 1).contiguous() for i in range(S)]
+    specs = [fbp.SliceSpec(W, fdeg, center, **kw) for _ in range(S)]
+    plan, wide = _run(specs, sinos, persistent=persistent)
+    assert plan.info(0)["tile_w"] == 32                                # the matrix-core items
+    plan.close()
+    _, one = _run(specs, sinos, slices_per_item=4, persistent=True)
+    for i in range(S):
+        rng = float(one[i].max() - one[i].min())
+        d = wide[i].astype(np.float64) - one[i]
+        assert np.sqrt(np.mean(d * d)) <= 2e-6 * rng and np.abs(d).max() <= 2e-5 * rng, (i, np.abs(d).max() / rng)
+    if not kw:
+        g = O.geometry(W, 2, center)
+        m = _circle(W, 0.4)
+        for i in (0, S - 1):
+            ref = O.recon_of64(sinos[i].numpy(), fdeg, g, O.set_filter(g.ndim, 0))
+            rms, _ = _errors(wide[i], ref, m)
+            rms1, _ = _errors(one[i], ref, m)
+            assert rms <= 2e-6 and rms <= 1.1 * rms1, (i, rms, rms1)
+
+
+def test_plan_matrix_core_stack_keeps_nonfinite_pixels():
+    """Samples that are not finite reach the pixels that they reach with one slice per
+    item, and no others: a NaN, an infinity and a finite row that overflows in the
+    filter, in three slices of a stack on the matrix cores."""
+    W, P, S = 640, 1221, 64
+    base, fdeg, c = _sino(W, P, 77, photons=1e4)
+    sinos = [torch.from_numpy(base).clone() for _ in range(S)]
+    sinos[3][700, 5] = float("nan")
+    sinos[17][0, W - 1] = float("inf")
+    sinos[63][P - 1] = 3e38
+    specs = [fbp.SliceSpec(W, fdeg, c) for _ in range(S)]
+    plan, wide = _run(specs, sinos, persistent=True)
+    assert plan.info(0)["tile_w"] == 32
+    plan.close()
+    _, one = _run(specs, sinos, slices_per_item=1)
+    for i in range(S):
+        assert np.array_equal(np.isfinite(wide[i]), np.isfinite(one[i])), i
+    assert 0 < np.isfinite(one[3]).mean() < 1          # an oblique row; slice 17's, at angle 0, covers the image
+    for i in (0, 2, 4, 62):
+        assert np.isfinite(wide[i]).all(), i
