@@ -240,8 +240,7 @@ static bool conv_wgrad(Unet* u, int li, const uint16_t* g, const uint16_t* x, in
     a.part = u->part;
     a.partb = u->part + (long long)a.nsplit * nw;
     return ok(launch_conv3x3_wgrad(a, s), "conv3x3 weight gradient") &&
-           ok(launch_sum_splits(a.part, a.nsplit, (int)nw, u->G + L.w, s), "sum") &&
-           ok(launch_sum_splits(a.partb, a.nsplit, L.cout, u->G + L.b, s), "sum");
+           ok(launch_sum_splits(a.part, a.nsplit, (int)nw, u->G + L.w, s, a.partb, L.cout, u->G + L.b), "sum");
 }
 
 // materialize: write the upsampled half of every concat (the backward pass
@@ -563,8 +562,7 @@ int rvConv3x3WgradBf16(const unsigned short* d_dy, int dy_stride, int dy_off, in
     a.part = part;
     a.partb = part + (long long)a.nsplit * nw;
     bool good = ok(launch_conv3x3_wgrad(a, s), "wgrad") &&
-                ok(launch_sum_splits(a.part, a.nsplit, (int)nw, d_dw, s), "sum");
-    if (good && d_db) good = ok(launch_sum_splits(a.partb, a.nsplit, Cout, d_db, s), "sum");
+                ok(launch_sum_splits(a.part, a.nsplit, (int)nw, d_dw, s, a.partb, d_db ? Cout : 0, d_db), "sum");
     good = good && ok(hipStreamSynchronize(s), "sync");
     (void)hipFree(part);
     return good ? 0 : -1;

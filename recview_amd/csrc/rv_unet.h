@@ -53,8 +53,9 @@ struct WgradArgs {
 };
 int wgrad_splits(int Cin, int Cout, int B, int H, int W);
 hipError_t launch_conv3x3_wgrad(const WgradArgs& a, hipStream_t s);
-// out[i] = sum_s part[s*n + i], i < n.
-hipError_t launch_sum_splits(const float* part, int nsplit, int n, float* out, hipStream_t s);
+// out[n] = column sums of part[nsplit][n]; with part2, out2[n2] = those of part2[nsplit][n2]
+hipError_t launch_sum_splits(const float* part, int nsplit, int n, float* out, hipStream_t s,
+                             const float* part2 = nullptr, int n2 = 0, float* out2 = nullptr);
 
 // Packs FP32 master weights W[Cout][9][Cin] into fragment order, for the
 // forward convolution (transpose = 0) or for its data gradient (transpose = 1:
