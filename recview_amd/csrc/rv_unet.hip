@@ -8,9 +8,8 @@
 //   weights (already in fragment order) in LDS, then each wave runs
 //   9 taps x 4 rows x NF fragments of MFMA.
 //   weight gradient: M = 16 output channels, N = 16 input channels, K = 32
-//   pixels.  Pixels are the contraction, so dY and X are staged transposed
-//   (pixel-contiguous) and X in three column-shifted copies, which keeps every
-//   fragment read an aligned 16-byte LDS load for all nine taps.
+//   pixels.  Pixels are the contraction; the LDS transpose reads turn the
+//   channel-contiguous dY and X into pixel-contiguous fragments.
 // Operand layouts (checked on gfx950): A[i][k] in lane i + 16*(k/8), element
 // k%8; B[k][j] in lane j + 16*(k/8), element k%8; D[i][j] in lane j + 16*(i/4),
 // element i%4.
@@ -545,97 +544,140 @@ hipError_t launch_conv3x3(const ConvArgs& a, hipStream_t s) {
 }
 
 // ------------------------------------------------------------ weight gradient
-constexpr int DY_PITCH = 144;   // bf16 per staged output channel: 128 pixels + 16 pad
-constexpr int XT_PITCH = 176;   // bf16 per staged (shift, channel): 10 x 16 pixels + 16 pad
+// One block: 16 * NFW output x 32 input channels, all nine taps, over the 8 x 16 pixel
+// patches split, split + nsplit, ...  dY and the halo of X are staged as they lie, one
+// LDS plane per 16 channels (32 bytes a pixel), and the LDS transpose read hands each
+// 16-lane group four pixels of 16 channels: a wave's read is one row of 16 pixels, 512
+// contiguous bytes, and a tap is only another address.  A contraction pairs the rows r
+// and r + 4, so the six row pairs of the halo serve all nine taps of all four pairs
+// from registers.  Bound by the LDS and by the latency of a patch's fetch, which the
+// second buffer hides.  Staged transposed instead, X in three shifted copies, 2-byte LDS
+// writes were most of the time: a layer of a 16 x 512^2 gradient took 266 us on average
+// with 64 and 539 us with 32 outputs per block, now 118 and 230 us.
+constexpr int WG_ROWS = 8;
+constexpr int DY_PLANE = 128 * 16 + 32;   // bf16 per plane: 128 pixels x 16 channels; the pads spread a
+constexpr int XT_PLANE = 180 * 16;        // thread group's writes over all banks (5760 bytes does)
+
+typedef short shortx4 __attribute__((ext_vector_type(4)));
+static __device__ __forceinline__ shortx4 lds_tr(const uint16_t* p) {
+    return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) shortx4*)p);
+}
+static __device__ __forceinline__ bf16x8 lds_tr2(const uint16_t* p, const uint16_t* q) {
+    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lds_tr(p), lds_tr(q), 0, 1, 2, 3, 4, 5, 6, 7));
+}
 
 template <int NFW>
-__global__ __launch_bounds__(256) void conv3x3_wgrad_kernel(WgradArgs a) {
-    constexpr int TCO = 16 * NFW;
-    constexpr int CF = NFW == 4 ? 2 : 1;
-    __shared__ __attribute__((aligned(16))) uint16_t dy_s[TCO * DY_PITCH];
-    __shared__ __attribute__((aligned(16))) uint16_t x_s[3 * 32 * XT_PITCH];
+__global__ __launch_bounds__(256, 2) void conv3x3_wgrad_kernel(WgradArgs a) {
+    constexpr int TCO = 16 * NFW, G = TCO / 8;
+    constexpr int CO = NFW / 2;                      // output fragments of a wave; one input fragment
+    constexpr int DYN = 128 * G / 256, XN = 3;       // 16-byte units of a thread
+    constexpr int BUF = NFW * DY_PLANE + 2 * XT_PLANE;
+    __shared__ __attribute__((aligned(16))) uint16_t lds[2 * BUF];
     const int t = threadIdx.x, l = t & 63, w = t >> 6;
     const int co0 = blockIdx.x * TCO, cc = blockIdx.y, split = blockIdx.z;
-    const int cof = w % NFW, cib = (w / NFW) * CF;
-    const int tiles_x = (a.W + 15) >> 4, tiles_y = (a.H + 7) >> 3;
+    const int cof = (w & 1) * CO, cif = w >> 1;
+    const int tiles_x = (a.W + 15) >> 4, tiles_y = (a.H + WG_ROWS - 1) / WG_ROWS;
     const int per_img = tiles_x * tiles_y, npatch = a.B * per_img;
-    floatx4 acc[9][CF];
+    floatx4 acc[9][CO];
 #pragma unroll
     for (int k = 0; k < 9; k++)
 #pragma unroll
-        for (int c = 0; c < CF; c++) acc[k][c] = floatx4{0.f, 0.f, 0.f, 0.f};
-    float bsum = 0.f;
-    for (int patch = split; patch < npatch; patch += a.nsplit) {
+        for (int c = 0; c < CO; c++) acc[k][c] = floatx4{0.f, 0.f, 0.f, 0.f};
+    float bsum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+
+    const int dg = t % G, dp = t / G;                // dY: channel group, first pixel
+    const int xg = t & 3, xp = t >> 2;               // X: channel group, first halo pixel
+    uint4 dv[DYN], xv[XN];
+    auto fetch = [&](int patch) {
         const int bb = patch / per_img, r = patch - bb * per_img;
-        const int y0 = (r / tiles_x) * 8, x0 = (r % tiles_x) * 16;
-        for (int i = t; i < 128 * (TCO / 8); i += 256) {
-            const int px = i / (TCO / 8), g = i - px * (TCO / 8);
-            const int y = y0 + (px >> 4), x = x0 + (px & 15);
-            uint4 v = make_uint4(0, 0, 0, 0);
-            if (y < a.H && x < a.W)
-                v = ld16(a.dy + (((long long)bb * a.H + y) * a.W + x) * a.dy_stride + a.dy_off + co0 +
-                         8 * g);
-            const uint16_t* e8 = (const uint16_t*)&v;
+        const int y0 = (r / tiles_x) * WG_ROWS, x0 = (r % tiles_x) * 16;
+        const long long img = (long long)bb * a.H;
 #pragma unroll
-            for (int e = 0; e < 8; e++) dy_s[(8 * g + e) * DY_PITCH + px] = e8[e];
+        for (int k = 0; k < DYN; k++) {
+            const int px = dp + k * (256 / G);
+            const int y = y0 + (px >> 4), x = x0 + (px & 15);
+            dv[k] = make_uint4(0, 0, 0, 0);
+            if (y < a.H && x < a.W) dv[k] = ld16(a.dy + ((img + y) * a.W + x) * a.dy_stride + a.dy_off + co0 + 8 * dg);
         }
-        for (int i = t; i < 720; i += 256) {
-            const int hp = i >> 2, g = i & 3;
+#pragma unroll
+        for (int k = 0; k < XN; k++) {
+            const int hp = xp + 64 * k;
             const int hy = hp / 18, hx = hp - hy * 18;
             const int y = y0 - 1 + hy, x = x0 - 1 + hx;
-            uint4 v = make_uint4(0, 0, 0, 0);
-            if (y >= 0 && y < a.H && x >= 0 && x < a.W)
-                v = ld16(a.x + (((long long)bb * a.H + y) * a.W + x) * a.x_stride + a.x_off + cc * 32 +
-                         8 * g);
-            const uint16_t* e8 = (const uint16_t*)&v;
+            xv[k] = make_uint4(0, 0, 0, 0);
+            if (hp < 180 && y >= 0 && y < a.H && x >= 0 && x < a.W)
+                xv[k] = ld16(a.x + ((img + y) * a.W + x) * a.x_stride + a.x_off + cc * 32 + 8 * xg);
+        }
+    };
+    int buf = 0;
+    if (split < npatch) fetch(split);
+    for (int patch = split; patch < npatch; patch += a.nsplit) {
+        uint16_t* dy_s = lds + buf;
+        uint16_t* x_s = dy_s + NFW * DY_PLANE;
 #pragma unroll
-            for (int kx = 0; kx < 3; kx++) {
-                const int c = hx - kx;
-                if (c < 0 || c >= 16) continue;
+        for (int k = 0; k < DYN; k++)
+            st16(dy_s + (dg >> 1) * DY_PLANE + (dp + k * (256 / G)) * 16 + 8 * (dg & 1), dv[k]);
 #pragma unroll
-                for (int e = 0; e < 8; e++) x_s[(kx * 32 + 8 * g + e) * XT_PITCH + hy * 16 + c] = e8[e];
+        for (int k = 0; k < XN; k++)
+            if (xp + 64 * k < 180) st16(x_s + (xg >> 1) * XT_PLANE + (xp + 64 * k) * 16 + 8 * (xg & 1), xv[k]);
+        if (cc == 0) {
+#pragma unroll
+            for (int k = 0; k < DYN; k++) {
+                const uint16_t* e8 = (const uint16_t*)&dv[k];
+#pragma unroll
+                for (int e = 0; e < 8; e++) bsum[e] += bf2f(e8[e]);
             }
         }
         __syncthreads();
-        if (cc == 0 && t < TCO) {
-            for (int px = 0; px < 128; px += 8) {
-                const uint4 v = ld16(dy_s + t * DY_PITCH + px);
-                const uint16_t* e8 = (const uint16_t*)&v;
+        if (patch + a.nsplit < npatch) fetch(patch + a.nsplit);
+        const uint16_t* xr = x_s + cif * XT_PLANE + 4 * l;
+        const uint16_t* dr = dy_s + cof * DY_PLANE + 4 * l;
+        bf16x8 bv[6][3];                             // halo rows r and r + 4, shift kx
+        auto rows = [&](int r) {
 #pragma unroll
-                for (int e = 0; e < 8; e++) bsum += bf2f(e8[e]);
-            }
-        }
-        const int q = l >> 4;
+            for (int kx = 0; kx < 3; kx++) bv[r][kx] = lds_tr2(xr + (r * 18 + kx) * 16, xr + ((r + 4) * 18 + kx) * 16);
+        };
+        rows(0);
+        rows(1);
 #pragma unroll
         for (int kb = 0; kb < 4; kb++) {
-            const bf16x8 av = *(const bf16x8*)(dy_s + (cof * 16 + (l & 15)) * DY_PITCH + kb * 32 + 8 * q);
-            const int rr = 2 * kb + (q >> 1), c0 = 8 * (q & 1);
+            rows(kb + 2);
+            bf16x8 av[CO];
 #pragma unroll
-            for (int tap = 0; tap < 9; tap++) {
-                const int ky = tap / 3, kx = tap % 3;
+            for (int c = 0; c < CO; c++)
+                av[c] = lds_tr2(dr + c * DY_PLANE + kb * 256, dr + c * DY_PLANE + (kb + 4) * 256);
 #pragma unroll
-                for (int cf = 0; cf < CF; cf++) {
-                    const int ci = (cib + cf) * 16 + (l & 15);
-                    const bf16x8 bv =
-                        *(const bf16x8*)(x_s + (kx * 32 + ci) * XT_PITCH + (rr + ky) * 16 + c0);
-                    acc[tap][cf] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv, acc[tap][cf], 0, 0, 0);
-                }
-            }
+            for (int tap = 0; tap < 9; tap++)
+#pragma unroll
+                for (int c = 0; c < CO; c++)
+                    acc[tap][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[c], bv[kb + tap / 3][tap % 3],
+                                                                          acc[tap][c], 0, 0, 0);
         }
-        __syncthreads();
+        buf = BUF - buf;
     }
     float* P = a.part + (long long)split * a.Cout * 9 * a.Cin;
 #pragma unroll
     for (int tap = 0; tap < 9; tap++)
 #pragma unroll
-        for (int cf = 0; cf < CF; cf++)
+        for (int c = 0; c < CO; c++)
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                const int co = co0 + cof * 16 + 4 * (l >> 4) + e;
-                const int ci = cc * 32 + (cib + cf) * 16 + (l & 15);
-                P[((long long)co * 9 + tap) * a.Cin + ci] = acc[tap][cf][e];
+                const int co = co0 + (cof + c) * 16 + 4 * (l >> 4) + e;
+                const int ci = cc * 32 + cif * 16 + (l & 15);
+                P[((long long)co * 9 + tap) * a.Cin + ci] = acc[tap][c][e];
             }
-    if (cc == 0 && t < TCO) a.partb[(long long)split * a.Cout + co0 + t] = bsum;
+    if (cc == 0) {
+        float* red = (float*)lds;
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < 8; e++) red[t * 8 + e] = bsum[e];
+        __syncthreads();
+        if (t < TCO) {
+            float s = 0.f;
+            for (int k = t / 8; k < 256; k += G) s += red[k * 8 + t % 8];
+            a.partb[(long long)split * a.Cout + co0 + t] = s;
+        }
+    }
 }
 
 int wgrad_splits(int Cin, int Cout, int B, int H, int W) {

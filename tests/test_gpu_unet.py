@@ -102,6 +102,26 @@ def test_conv_weight_gradient(cin, cout, H, W):
     assert rel(db.double().cpu().numpy(), rb) < 1e-5
 
 
+@pytest.mark.parametrize("cin,cout,B,H,W", [
+    (32, 32, 1, 2, 2),           # one patch, mostly empty
+    (64, 32, 1, 9, 17),          # one row and one column past a patch
+    (32, 32, 3, 130, 325),       # 1071 patches for 1024 splits: some splits walk two
+    (256, 256, 2, 41, 63),       # 32 splits of 48 patches
+    (32, 64, 1, 200, 24)])       # 16 to 127 splits
+def test_conv_weight_gradient_splits(cin, cout, B, H, W):
+    """Patch remainders and split counts of the weight gradient against the FP64 oracle:
+    FP32 sums of at most 65000 products, rounding errors of random sign, so well below
+    sqrt(65000) / 2 * 2^-24 = 7.6e-6 of the result's RMS."""
+    rng = np.random.default_rng(cin + cout + H)
+    g = U.bf16_round(rng.standard_normal((B, H, W, cout)))
+    x = U.bf16_round(rng.standard_normal((B, H, W, cin)))
+    dw, db = RU.conv3x3_wgrad(bf(g), bf(x), cin, cout, (B, H, W))
+    torch.cuda.synchronize()
+    rw, rb = U.conv3x3_wgrad(g, x)
+    assert rel(dw.double().cpu().numpy(), rw) < 1e-5
+    assert rel(db.double().cpu().numpy(), rb) < 1e-5
+
+
 def _images(rng, B, H, W):
     """Smooth random images with edges, like reconstructed slices."""
     x = rng.standard_normal((B, H, W))
