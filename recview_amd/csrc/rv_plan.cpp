@@ -73,6 +73,7 @@ struct Group {
     int* d_order = nullptr;
     int total_items = 0;
     int grid = 0;
+    int parts = 0;               // workgroups per tile (bp_sub_parts), 0: persistent or one per tile
 };
 
 }  // namespace
@@ -328,6 +329,11 @@ int launch_backprojection(rv_plan_t p, hipStream_t st, bool pack = true)
             L.counter = ctr;
             L.part = p->d_xsum;
             rv::launch_bpx(L, G.grid, st);
+            continue;
+        }
+        if (G.parts) {
+            L.counter = nullptr;
+            rv::launch_bp_sub(L, G.parts, st);
             continue;
         }
         if (L.counter) rv::launch_zero_u32(ctr, rv::kXcds * rv::kCounterStride, st);
@@ -845,6 +851,7 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
             x_grid = std::max(x_grid, G.grid);
             continue;
         }
+        G.parts = rv::bp_sub_parts(G.mode, G.tile, G.total_items);
         (void)rv::bp_blocks_per_cu_tg(G.mode, G.tile, G.chunk, G.tgeom);     // sets LDS attributes outside capture
         if (opt->persistent) {
             const int per_cu = rv::bp_blocks_per_cu_tg(G.mode, G.tile, G.chunk, G.tgeom);

@@ -772,3 +772,27 @@ def test_plan_matrix_core_stack_keeps_nonfinite_pixels():
     assert 0 < np.isfinite(one[3]).mean() < 1          # an oblique row; slice 17's, at angle 0, covers the image
     for i in (0, 2, 4, 62):
         assert np.isfinite(wide[i]).all(), i
+
+
+@pytest.mark.parametrize("W,P,k,store,dtype", [(40, 7, 1, "f32", "f32"), (130, 64, 1, "bf16", "f32"),
+                                               (520, 33, 1, "f32", "i16"), (700, 31, 1, "f16", "f32"),
+                                               (65, 33, 2, "f32", "f32"), (200, 48, 4, "f32", "f32"),
+                                               (601, 17, 4, "f32", "f32"), (900, 16, 2, "f32", "f32")])
+def test_plan_parts_of_tiles_equal_whole_tiles(W, P, k, store, dtype):
+    """Launches of few tiles split each over several workgroups: the images are those
+    of whole tiles bit for bit (the same slices beside others that fill the launch)."""
+    print(f"case {W} x {P}, {k} per item, {store} {dtype}", flush=True)
+    specs, sinos = [], []
+    for i in range(k):
+        s, fdeg, c = _sino(W, P, 3100 + i)
+        x = torch.from_numpy(s)
+        specs.append(fbp.SliceSpec(W, fdeg, c, sino_dtype=dtype))
+        sinos.append(phantom.to_int16(x) if dtype == "i16" else x)
+    fill = [fbp.SliceSpec(1800, np.array([0.0, 90.0], np.float32), 900.3, sino_dtype=dtype) for _ in range(k)]
+    rows = [torch.zeros(2, 1800, dtype=sinos[0].dtype) for _ in range(k)]
+    _, few = _run(specs, sinos, store=store)
+    for persistent in (False, True):
+        _, many = _run(specs + fill, sinos + rows, store=store, persistent=persistent)
+        for i in range(k):
+            assert np.array_equal(few[i], many[i]), (i, persistent)
+    assert np.abs(few[0]).max() > 0
