@@ -172,6 +172,12 @@ int RecviewSinogramDevice(const unsigned short* d_frames, int nframes, int mult,
                           const float* fexp, const float* fdeg, unsigned flags, int drStart, int drEnd,
                           double drX, double drY, int drOmit, const int* piDrift, int is8bit, int start,
                           int step, int binning, int out_float, void* d_out, rv_stream_t stream);
+/* The same into a d_out of any contents, which is written whole: rows that are not
+ * converted become zero. */
+int RecviewSinogramDeviceZero(const unsigned short* d_frames, int nframes, int mult, int W, const char* binc,
+                              const float* fexp, const float* fdeg, unsigned flags, int drStart, int drEnd,
+                              double drX, double drY, int drOmit, const int* piDrift, int is8bit, int start,
+                              int step, int binning, int out_float, void* d_out, rv_stream_t stream);
 
 /* ------------------------------------------ Part 1: kernel wrappers -- */
 

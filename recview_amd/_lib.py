@@ -76,6 +76,7 @@ EXPORTS = [
     "rvUnetCreate", "rvUnetParamCount", "rvUnetGetParams", "rvUnetSetParams", "rvUnetForward",
     "rvUnetLossGrad", "rvUnetTrainStep", "rvUnetDestroy", "rvConv3x3Bf16", "rvConv3x3WgradBf16",
     "RecviewOutputStage", "RecviewImageDescription", "RecviewWriteTif16", "RecviewSinogramDevice",
+    "RecviewSinogramDeviceZero",
     "RecviewDeviceAlloc", "RecviewDeviceFree", "RecviewCopyToHost", "RecviewCopyToDevice",
     "RecviewOutputStageNoAlloc",
 ]
@@ -139,6 +140,7 @@ def _declare(L):
     L.RecviewSinogramDevice.argtypes = [vp, C.c_int, C.c_int, C.c_int, C.c_char_p, fp, fp, C.c_uint, C.c_int,
                                         C.c_int, C.c_double, C.c_double, C.c_int, ip, C.c_int, C.c_int,
                                         C.c_int, C.c_int, C.c_int, vp, vp]
+    L.RecviewSinogramDeviceZero.argtypes = L.RecviewSinogramDevice.argtypes
     L.RecviewOutputStage.argtypes = [vp, C.c_int, C.c_int, C.c_double, C.c_int, vp, C.POINTER(C.c_double),
                                      C.POINTER(C.c_double), vp]
     L.RecviewOutputStageNoAlloc.argtypes = [vp, C.c_int, C.c_int, C.c_double, C.c_int, vp, vp, vp]

@@ -513,13 +513,11 @@ bool sinogram_jobs(const SinoWalk& w, std::vector<SinoJob>& jobs)
         }
         if (action == 1 && (binc[i] & CGAZODOC_BINC_SKIP)) action = 2;
         if (action == 1 && (w.flags & RQFLAGS_DRIFTLIST) && w.piDrift) idrift -= w.piDrift[i];
-        for (int k = 0; k < w.mult; k++) {
-            SinoJob J{};
-            J.frame = i; J.k = k; J.i0 = i0; J.i1 = i1; J.t0 = t0;
-            J.shift = action == 1 ? idrift / w.binning : 0;
-            J.action = action;
-            jobs.push_back(J);
-        }
+        SinoJob J{};
+        J.frame = i; J.i0 = i0; J.i1 = i1; J.t0 = t0;
+        J.shift = action == 1 ? idrift / w.binning : 0;
+        J.action = action;
+        jobs.push_back(J);
     }
     return true;
 }
@@ -528,10 +526,10 @@ bool sinogram_jobs(const SinoWalk& w, std::vector<SinoJob>& jobs)
 
 extern "C" {
 
-int RecviewSinogramDevice(const unsigned short* d_frames, int nframes, int mult, int W, const char* binc,
-                          const float* fexp, const float* fdeg, unsigned flags, int drStart, int drEnd,
-                          double drX, double drY, int drOmit, const int* piDrift, int is8bit, int start,
-                          int step, int binning, int out_float, void* d_out, rv_stream_t stream)
+static int sinogram_device(const unsigned short* d_frames, int nframes, int mult, int W, const char* binc,
+                           const float* fexp, const float* fdeg, unsigned flags, int drStart, int drEnd,
+                           double drX, double drY, int drOmit, const int* piDrift, int is8bit, int start,
+                           int step, int binning, int out_float, void* d_out, rv_stream_t stream, bool zero_others)
 {
     if (!d_frames || !d_out || !binc || !fexp || !fdeg || nframes < 2 || mult <= 0 || W <= 0 || step <= 0 ||
         binning <= 0) {
@@ -545,6 +543,18 @@ int RecviewSinogramDevice(const unsigned short* d_frames, int nframes, int mult,
     walk.start = start; walk.step = step; walk.binning = binning;
     std::vector<rv::SinoJob> jobs;
     const bool good_walk = rv::sinogram_jobs(walk, jobs);
+    const size_t converted = jobs.size();
+    if (zero_others) {
+        // the converted frames come in ascending order
+        size_t q = 0;
+        for (int i = 0; i < nframes; i++) {
+            if (q < converted && jobs[q].frame == i) { q++; continue; }
+            rv::SinoJob J{};
+            J.frame = i;
+            J.action = 2;
+            jobs.push_back(J);
+        }
+    }
     if (!jobs.empty()) {
         hipStream_t s = (hipStream_t)stream;
         rv::SinoJob* d_jobs = nullptr;
@@ -563,7 +573,25 @@ int RecviewSinogramDevice(const unsigned short* d_frames, int nframes, int mult,
         rv::set_message("RecviewSinogramDevice: no incident frame for a sample frame");
         return -2;
     }
-    return (int)jobs.size();
+    return (int)converted * mult;
+}
+
+int RecviewSinogramDevice(const unsigned short* d_frames, int nframes, int mult, int W, const char* binc,
+                          const float* fexp, const float* fdeg, unsigned flags, int drStart, int drEnd,
+                          double drX, double drY, int drOmit, const int* piDrift, int is8bit, int start,
+                          int step, int binning, int out_float, void* d_out, rv_stream_t stream)
+{
+    return sinogram_device(d_frames, nframes, mult, W, binc, fexp, fdeg, flags, drStart, drEnd, drX, drY, drOmit,
+                           piDrift, is8bit, start, step, binning, out_float, d_out, stream, false);
+}
+
+int RecviewSinogramDeviceZero(const unsigned short* d_frames, int nframes, int mult, int W, const char* binc,
+                              const float* fexp, const float* fdeg, unsigned flags, int drStart, int drEnd,
+                              double drX, double drY, int drOmit, const int* piDrift, int is8bit, int start,
+                              int step, int binning, int out_float, void* d_out, rv_stream_t stream)
+{
+    return sinogram_device(d_frames, nframes, mult, W, binc, fexp, fdeg, flags, drStart, drEnd, drX, drY, drOmit,
+                           piDrift, is8bit, start, step, binning, out_float, d_out, stream, true);
 }
 
 void CudaSinogramHost(RECONST_INFO* ri, int idev, bool)
@@ -598,7 +626,7 @@ void CudaSinogramHost(RECONST_INFO* ri, int idev, bool)
     if (!jobs.empty()) {
         if (!rv::hip_ok(hipSetDevice(idev), "hipSetDevice")) { ri->iStatus = RECONST_INFO_ERROR; return; }
         const size_t nrow = (size_t)isino * M, frame_bytes = nrow * W * sizeof(uint16_t);
-        const size_t out_bytes = jobs.size() * W * sizeof(int16_t);
+        const size_t out_bytes = jobs.size() * M * W * sizeof(int16_t);
         uint16_t *h_frames = nullptr, *d_frames = nullptr;
         int16_t *h_out = nullptr, *d_out = nullptr;
         rv::SinoJob* d_jobs = nullptr;
@@ -623,8 +651,8 @@ void CudaSinogramHost(RECONST_INFO* ri, int idev, bool)
                        rv::hip_ok(hipStreamSynchronize(st), "sync");
             }
             if (good)
-                for (size_t q = 0; q < jobs.size(); q++)
-                    std::memcpy(ri->iSinogr[(size_t)jobs[q].frame * M + jobs[q].k], h_out + q * W,
+                for (size_t q = 0; q < jobs.size() * M; q++)
+                    std::memcpy(ri->iSinogr[(size_t)jobs[q / M].frame * M + q % M], h_out + q * W,
                                 W * sizeof(int16_t));
         }
         if (st) (void)hipStreamDestroy(st);

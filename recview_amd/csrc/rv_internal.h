@@ -66,12 +66,12 @@ void launch_bp_lut_global(int* d_ifp, const int* d_igp, int N, float fcos, float
                           float foffset, int rule, int block, hipStream_t stream);
 
 // ------------------------------------------------------- sinogram generation
-// One converted row: frame `frame`, multiplex line k, incident frames i0 / i1
-// with weight t0, drift shift (samples), action 1 = convert, 2 = zero.
+// One converted frame (all its multiplex lines): incident frames i0 / i1 with
+// weight t0, drift shift (samples), action 1 = convert, 2 = zero.
 struct SinoJob {
-    int frame, k, i0, i1;
+    int frame, i0, i1;
     float t0;
-    int shift, action, pad;
+    int shift, action;
 };
 void launch_sinogram(const uint16_t* frames, int nframes, int mult, int W, const SinoJob* jobs,
                      int njobs, void* out, int pixmin, int zernike, int out_float, int out_full,

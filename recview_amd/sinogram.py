@@ -56,16 +56,18 @@ def generate_device(frames, binc, fexp, fdeg, flags=0, drift=(0, 0, 0.0, 0.0, 0)
     if frames.dtype != torch.int16 or not frames.is_cuda or frames.dim() != 3:
         raise ValueError("frames must be an int16 device tensor [nframes][mult][W]")
     nframes, mult, W = frames.shape
+    convert = _lib.lib().RecviewSinogramDevice
     if out is None:
-        out = torch.zeros(nframes, mult, W, dtype=torch.float32 if out_float else torch.int16,
+        out = torch.empty(nframes, mult, W, dtype=torch.float32 if out_float else torch.int16,
                           device=frames.device)
+        convert = _lib.lib().RecviewSinogramDeviceZero      # clears the rows that are not converted
     binc = np.ascontiguousarray(binc, np.int8)
     fexp = np.ascontiguousarray(fexp, np.float32)
     fdeg = np.ascontiguousarray(fdeg, np.float32)
     pd = None if pidrift is None else np.ascontiguousarray(pidrift, np.int32)
     drs, dre, dx, dy, om = drift
     s = stream if stream is not None else torch.cuda.current_stream()
-    n = _lib.lib().RecviewSinogramDevice(
+    n = convert(
         C.c_void_p(frames.contiguous().data_ptr()), nframes, mult, W, binc.ctypes.data_as(C.c_char_p),
         fexp.ctypes.data_as(C.POINTER(C.c_float)), fdeg.ctypes.data_as(C.POINTER(C.c_float)), int(flags),
         int(drs), int(dre), float(dx), float(dy), int(om),

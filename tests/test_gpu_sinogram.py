@@ -108,3 +108,39 @@ def test_device_frames_float_rows():
     assert np.abs(expect - q).max() <= 1
     assert np.mean(expect != q) < 1e-3
     assert (np.abs(f[:-1][~conv]) == 0).all()                 # incident / dark rows untouched
+
+
+@pytest.mark.parametrize("W,mult", [(1, 1), (7, 3), (8, 1), (300, 2), (2048, 1), (2056, 2), (4099, 1)])
+def test_device_frames_row_widths(W, mult):
+    """Rows around the 8-sample loads and the 2048-sample blocks, and unaligned frames:
+    int16 rows equal the host conversion, float rows the 64-bit logarithm rounded to
+    FP32 (to one unit in the last place), rows that are not converted are zero."""
+    import torch
+    print(f"case W={W} mult={mult}", flush=True)
+    frames, binc, fexp, fdeg = _scan(51 + W, mult=mult, W=W)
+    host, _ = sinogram.generate(frames, binc, fexp, fdeg)
+    buf = torch.empty(frames.size + 1, dtype=torch.int16, device="cuda")
+    conv = np.zeros(frames.shape[0], bool)
+    conv[:-1] = (binc[:-1] & 1) != 0
+    inc = np.nonzero(binc[:-1] == 0)[0]
+    f = frames.astype(np.int64)
+    ref = np.zeros(frames.shape)
+    for i in np.nonzero(conv)[0]:
+        i0 = inc[inc < i][-1]
+        i1 = inc[inc > i][0] if (inc > i).any() else i0
+        t = np.float32(0) if i0 == i1 else (fexp[i] - fexp[i0]) / (fexp[i1] - fexp[i0])
+        w = f[i0].astype(np.float32) + (f[i1] - f[i0]).astype(np.float32) * np.float32(t) - f[-1].astype(np.float32)
+        s = f[i] - f[-1]
+        ok = (w > 0) & (s >= 20)
+        ref[i][ok] = np.log(w.astype(np.float64)[ok] / s[ok])
+    for off in (0, 1):
+        d = buf[off:off + frames.size].view(frames.shape)
+        d.copy_(torch.from_numpy(frames.view(np.int16)))
+        if off:
+            assert d.data_ptr() % 16 != 0
+        rows, _ = sinogram.generate_device(d, binc, fexp, fdeg, out_float=False)
+        assert np.array_equal(rows.cpu().numpy()[conv], host[conv])
+        assert (rows.cpu().numpy()[~conv] == 0).all()
+        rows, _ = sinogram.generate_device(d, binc, fexp, fdeg)
+        got = rows.cpu().numpy()
+        assert (np.abs(got - ref.astype(np.float32)) <= np.spacing(np.abs(ref).astype(np.float32))).all()
