@@ -57,9 +57,11 @@ class ReconstInfo:
     def set_rows(self, rows_i16):
         rows = np.ascontiguousarray(rows_i16, np.int16)
         self._rows = rows
+        # the row pointers as one array of addresses (with a ctypes pointer object per
+        # row, a call for 2048^2 x 1800 took 9.9 ms instead of 3.6)
+        addr = rows.ctypes.data + np.arange(rows.shape[0], dtype=np.uintp) * rows.strides[0]
         ptrs = (C.POINTER(C.c_short) * rows.shape[0])()
-        for i in range(rows.shape[0]):
-            ptrs[i] = rows[i].ctypes.data_as(C.POINTER(C.c_short))
+        C.memmove(ptrs, addr.ctypes.data, addr.nbytes)
         self._ptrs = ptrs
         self.ri.iSinogr = C.cast(ptrs, C.POINTER(C.POINTER(C.c_short)))
         self.ri.maxSinogrLen = rows.shape[0]
