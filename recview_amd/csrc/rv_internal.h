@@ -95,14 +95,11 @@ bool sinogram_jobs(const SinoWalk& w, std::vector<SinoJob>& jobs);
 
 // ------------------------------------------------------- output stage
 // Min/max + normalisation to 0..65534 inside the circle of squared radius
-// irad2 (gazoDoc.cpp:3993-4021).  scratch: >= 2050 elements of the image type;
-// its last two hold (min, max) afterwards.
-void launch_output_stage(const void* img, int is_float, int N, int irad2, uint16_t* out, void* scratch,
-                         hipStream_t s);
-// The same three launches with the 1024 partial minima and 1024 partial maxima at
-// part (2048 values of the image type) and the (min, max) result at range.
+// irad2 (gazoDoc.cpp:3993-4021).  part: room for 1024 partial minima and 1024 partial
+// maxima (values of the image type); (min, max) are written to range.
 void launch_output_stage_parts(const void* img, int is_float, int N, int irad2, uint16_t* out, void* part,
                                void* range, hipStream_t s);
+void drop_output_work(int dev);
 constexpr int kOutputParts = 1024;
 // Squared mask radius of gazoDoc.cpp:4008-4010: r = zoom * center / binning,
 // min(r, N - r) truncated, for the zoom and binning of iInterpolation.

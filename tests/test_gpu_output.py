@@ -32,6 +32,27 @@ def test_output_stage_bit_exact(N, interp, center, lo, hi):
         assert (fmin, fmax) == (rmin, rmax)
 
 
+@pytest.mark.parametrize("N,offset", [(1, 0), (2, 0), (3, 1), (64, 2), (91, 0), (130, 3), (300, 0), (1500, 0), (2051, 1)])
+def test_output_stage_sides_and_alignment(N, offset):
+    """Sides around the 4-pixel groups and the partials of a workgroup, images that start
+    on any value, extremes at both ends; NaN is passed over."""
+    rng = np.random.default_rng(N)
+    img = rng.integers(-3000, 90000, (N, N)).astype(np.int32)
+    img[0, 0], img[-1, -1] = -70000, 200000
+    for dt in (torch.int32, torch.float32):
+        buf = torch.empty(N * N + offset, dtype=dt, device="cuda")
+        d = buf[offset:].view(N, N)
+        d.copy_(torch.from_numpy(img))
+        ref, rmin, rmax = O.output_stage(img, 1, N / 2 + 0.3, 1)
+        got, gmin, gmax = output.output_stage(d, N / 2 + 0.3)
+        assert (gmin, gmax) == (rmin, rmax), dt
+        assert np.array_equal(got.cpu().numpy().view(np.uint16).astype(np.int32), ref), dt
+    if N > 2:
+        d[N // 2, 0] = float("nan")
+        _, gmin, gmax = output.output_stage(d, N / 2 + 0.3)
+        assert (gmin, gmax) == (rmin, rmax)
+
+
 def test_slice_to_tif(tmp_path):
     rng = np.random.default_rng(3)
     img = rng.normal(0, 1, (128, 128)).astype(np.float32)
