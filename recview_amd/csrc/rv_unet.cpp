@@ -308,9 +308,9 @@ static bool backward(Unet* u, hipStream_t s) {
     const int B = u->B, H = u->H, W = u->W;
     const int nb = edge_blocks(B, H, W);
     const ULayer& Lo = u->layers[u->li_out()];
-    if (!ok(launch_edge_out_wgrad(u->dy, u->d[0], u->C(0), u->part, nb, B, H, W, s), "edge grad") ||
-        !ok(launch_sum_splits(u->part, nb, 9 * u->C(0) + 1, u->G + Lo.w, s), "sum") ||
-        !ok(launch_edge_out_bwd(u->dy, u->P + Lo.w, u->d[0], u->C(0), u->g_d[0], B, H, W, s), "edge grad"))
+    if (!ok(launch_edge_out_grad(u->dy, u->d[0], u->C(0), u->P + Lo.w, u->g_d[0], u->part, nb, B, H, W, s),
+            "edge grad") ||
+        !ok(launch_sum_splits(u->part, nb, 9 * u->C(0) + 1, u->G + Lo.w, s), "sum"))
         return false;
     for (int l = 0; l <= Lv - 2; l++) {
         const int db = u->li_dec(l, 1), dA = u->li_dec(l, 0);

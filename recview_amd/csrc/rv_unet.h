@@ -73,12 +73,10 @@ hipError_t launch_edge_in_wgrad(const uint16_t* dy, int C, const float* x, float
 // Last layer: y[p] = xres[p] + b + sum W[tap][c] * X[p + d(tap)][c]  (C -> 1, fp32 out).
 hipError_t launch_edge_out(const uint16_t* x, int C, const float* w, const float* b,
                            const float* xres, float* y, int B, int H, int W, hipStream_t s);
-// dX[p][c] = (X[p][c] > 0) * sum_tap W[tap][c] * dy[p - d(tap)]
-hipError_t launch_edge_out_bwd(const float* dy, const float* w, const uint16_t* x, int C,
-                               uint16_t* dx, int B, int H, int W, hipStream_t s);
-// part[blk][tap*C + c] (9*C entries) and part[blk][9*C] = sum dy.
-hipError_t launch_edge_out_wgrad(const float* dy, const uint16_t* x, int C, float* part, int nblk,
-                                 int B, int H, int W, hipStream_t s);
+// dX[p][c] = (X[p][c] > 0) * sum_tap W[tap][c] * dy[p - d(tap)], and
+// part[blk][tap*C + c] (9*C entries), part[blk][9*C] = sum dy.
+hipError_t launch_edge_out_grad(const float* dy, const uint16_t* x, int C, const float* w, uint16_t* dx,
+                                float* part, int nblk, int B, int H, int W, hipStream_t s);
 
 // 2x2 average pooling (H, W: input size), nearest 2x upsampling into a
 // channel slice of a wider tensor (H, W: output size) and its gradient.

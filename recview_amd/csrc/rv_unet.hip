@@ -843,59 +843,124 @@ int edge_blocks(int B, int H, int W) {
     return (int)std::max(1LL, std::min(1024LL, (n + 4095) / 4096));
 }
 
-// Pixels of block k: [k*ppb, min(n, (k+1)*ppb)).  Thread t handles channel
-// group t % (C/8) for every (256 / (C/8))-th pixel.  part[blk] = weights
-// [c][tap] (9*C) then biases [c] (C), the layout of the parameters.
-template <int C>
-__global__ void edge_in_wgrad_kernel(const uint16_t* dy, const float* x, float* part, int B, int H,
-                                     int W) {
-    constexpr int G = C / 8, LANES = 256 / G;
-    __shared__ float red[C * 10];
-    const long long n = (long long)B * H * W;
-    const long long ppb = (n + gridDim.x - 1) / gridDim.x;
-    const long long p0 = blockIdx.x * ppb, p1 = p0 + ppb < n ? p0 + ppb : n;
+// Gradients of the two edge layers, whose one side is an image v (the input, or dy of the
+// output layer) and whose other side is activations c of C channels: every pixel's C
+// channels against the 3 x 3 neighbours in v,
+//   first layer: dW[c][tap] = sum_p dy[p][c] x[p + d(tap)], dB[c] = sum_p dy[p][c];
+//   last layer (OUT): dW[tap][c] = sum_p X[p][c] dy[p - d(tap)], dB = sum_p dy[p], and on
+//   the way dX[p][c] = (X[p][c] > 0) sum_tap W[tap][c] dy[p - d(tap)].
+// Bound by the activations: each is read once, the neighbours move down a strip of
+// 256 / (C / 8) columns x kEdgeRows rows in registers (three loads a row), and the
+// activations of the next row load meanwhile.  Thread t handles channel group t % (C / 8).
+// part[blk]: the layout of the parameters, sums of the strips blk, blk + gridDim.x, ...
+// 16 x 512^2 x 32: last layer 350 us (each activation read for nine taps) and 240 us for
+// dX apart -> 227 us in one; first layer 196 -> 92 us.
+constexpr int kEdgeRows = 8;
+
+template <int C, bool OUT>
+__global__ __launch_bounds__(256) void edge_grad_kernel(const float* v, const uint16_t* c, const float* w,
+                                                        uint16_t* dx, float* part, int B, int H, int W) {
+    constexpr int G = C / 8, LANES = 256 / G, NB = OUT ? 9 * C + 1 : 10 * C;
+    __shared__ float red[4][10 * C];
     const int t = threadIdx.x, g = t % G;
-    float acc[8][10];
+    float acc[9][8], bs[8], wr[OUT ? 9 : 1][8];
 #pragma unroll
-    for (int e = 0; e < 8; e++)
-#pragma unroll
-        for (int k = 0; k < 10; k++) acc[e][k] = 0.f;
-    for (int i = t; i < C * 10; i += 256) red[i] = 0.f;
-    for (long long p = p0 + t / G; p < p1; p += LANES) {
-        int bb, y, xx;
-        pix_coords(p, H, W, bb, y, xx);
-        const uint4 d = ld16(dy + p * C + 8 * g);
-        const uint16_t* d8 = (const uint16_t*)&d;
-        float v[9];
-#pragma unroll
-        for (int tap = 0; tap < 9; tap++) {
-            const int yy = y + tap / 3 - 1, x2 = xx + tap % 3 - 1;
-            v[tap] = (yy >= 0 && yy < H && x2 >= 0 && x2 < W) ? x[((long long)bb * H + yy) * W + x2] : 0.f;
-        }
+    for (int k = 0; k < 9; k++)
 #pragma unroll
         for (int e = 0; e < 8; e++) {
-            const float de = bf2f(d8[e]);
+            acc[k][e] = 0.f;
+            if constexpr (OUT) wr[k][e] = w[k * C + 8 * g + e];
+        }
 #pragma unroll
-            for (int tap = 0; tap < 9; tap++) acc[e][tap] = fmaf(de, v[tap], acc[e][tap]);
-            acc[e][9] += de;
+    for (int e = 0; e < 8; e++) bs[e] = 0.f;
+    const int ncol = (W + LANES - 1) / LANES, nrow = (H + kEdgeRows - 1) / kEdgeRows;
+    for (int s = blockIdx.x; s < B * nrow * ncol; s += gridDim.x) {
+        const int x = s % ncol * LANES + t / G, y0 = s / ncol % nrow * kEdgeRows;
+        const int y1 = min(H, y0 + kEdgeRows);
+        const long long img = (long long)(s / ncol / nrow) * H * W;
+        float win[3][3];
+        auto load_row = [&](int y, float (&r)[3]) {
+#pragma unroll
+            for (int k = 0; k < 3; k++) {
+                const int xx = x + k - 1;
+                r[k] = (y >= 0 && y < H && xx >= 0 && xx < W) ? v[img + (long long)y * W + xx] : 0.f;
+            }
+        };
+        auto load_c = [&](int y) {
+            uint4 q = {0, 0, 0, 0};
+            if (x < W && y < y1) q = ld16(c + (img + (long long)y * W + x) * C + 8 * g);
+            return q;
+        };
+        load_row(y0 - 1, win[0]);
+        load_row(y0, win[1]);
+        uint4 next = load_c(y0);
+        for (int y = y0; y < y1; y++) {
+            load_row(y + 1, win[2]);
+            const uint4 cur = next;
+            next = load_c(y + 1);
+            const uint16_t* c8 = (const uint16_t*)&cur;
+            // the neighbour of a tap: p + d(tap), for the last layer p - d(tap)
+            auto nb = [&](int tap) { return OUT ? win[2 - tap / 3][2 - tap % 3] : win[tap / 3][tap % 3]; };
+            uint4 r;
+            uint16_t* r8 = (uint16_t*)&r;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const float a = bf2f(c8[e]);
+#pragma unroll
+                for (int tap = 0; tap < 9; tap++) acc[tap][e] = fmaf(a, nb(tap), acc[tap][e]);
+                if constexpr (OUT) {
+                    float d = 0.f;
+#pragma unroll
+                    for (int tap = 0; tap < 9; tap++) d = fmaf(wr[tap][e], nb(tap), d);
+                    r8[e] = f2bf(a > 0.f ? d : 0.f);
+                } else {
+                    bs[e] += a;
+                }
+            }
+            if constexpr (OUT) {
+                if (x < W) {
+                    bs[0] += win[1][1];
+                    st16(dx + (img + (long long)y * W + x) * C + 8 * g, r);
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < 3; k++) {
+                win[0][k] = win[1][k];
+                win[1][k] = win[2][k];
+            }
+        }
+    }
+    auto sum = [&](float a) {
+        for (int off = 32; off >= G; off >>= 1) a += __shfl_xor(a, off);
+        return a;
+    };
+    float* mine = red[t >> 6];
+    const bool first = (t & 63) < G;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+#pragma unroll
+        for (int k = 0; k < 9; k++) {
+            const float a = sum(acc[k][e]);
+            if (first) mine[OUT ? k * C + 8 * g + e : (8 * g + e) * 9 + k] = a;
+        }
+        if (!OUT || e == 0) {
+            const float a = sum(bs[e]);
+            if (first && (!OUT || g == 0)) mine[9 * C + (OUT ? 0 : 8 * g + e)] = a;
         }
     }
     __syncthreads();
-#pragma unroll
-    for (int e = 0; e < 8; e++)
-#pragma unroll
-        for (int k = 0; k < 10; k++)
-            atomicAdd(&red[k < 9 ? (8 * g + e) * 9 + k : 9 * C + 8 * g + e], acc[e][k]);
-    __syncthreads();
-    for (int i = t; i < C * 10; i += 256) part[(long long)blockIdx.x * C * 10 + i] = red[i];
+    for (int i = t; i < NB; i += 256)
+        part[(long long)blockIdx.x * NB + i] = (red[0][i] + red[1][i]) + (red[2][i] + red[3][i]);
 }
 
 hipError_t launch_edge_in_wgrad(const uint16_t* dy, int C, const float* x, float* part, int nblk,
                                 int B, int H, int W, hipStream_t s) {
     if (C == 32)
-        hipLaunchKernelGGL(edge_in_wgrad_kernel<32>, dim3(nblk), dim3(256), 0, s, dy, x, part, B, H, W);
+        hipLaunchKernelGGL((edge_grad_kernel<32, false>), dim3(nblk), dim3(256), 0, s, x, dy, nullptr, nullptr, part,
+                           B, H, W);
     else if (C == 64)
-        hipLaunchKernelGGL(edge_in_wgrad_kernel<64>, dim3(nblk), dim3(256), 0, s, dy, x, part, B, H, W);
+        hipLaunchKernelGGL((edge_grad_kernel<64, false>), dim3(nblk), dim3(256), 0, s, x, dy, nullptr, nullptr, part,
+                           B, H, W);
     else
         return hipErrorInvalidValue;
     return hipGetLastError();
@@ -952,97 +1017,12 @@ hipError_t launch_edge_out(const uint16_t* x, int C, const float* w, const float
     return hipGetLastError();
 }
 
-template <int C>
-__global__ void edge_out_bwd_kernel(const float* dy, const float* w, const uint16_t* x, uint16_t* dx,
-                                    int B, int H, int W) {
-    const long long p = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (p >= (long long)B * H * W) return;
-    int bb, yy, xx;
-    pix_coords(p, H, W, bb, yy, xx);
-    float d[9];
-#pragma unroll
-    for (int tap = 0; tap < 9; tap++) {
-        const int y2 = yy - (tap / 3 - 1), x2 = xx - (tap % 3 - 1);
-        d[tap] = (y2 >= 0 && y2 < H && x2 >= 0 && x2 < W) ? dy[((long long)bb * H + y2) * W + x2] : 0.f;
-    }
-#pragma unroll
-    for (int g = 0; g < C / 8; g++) {
-        const uint4 xv = ld16(x + p * C + 8 * g);
-        const uint16_t* x8 = (const uint16_t*)&xv;
-        uint4 r;
-        uint16_t* r8 = (uint16_t*)&r;
-#pragma unroll
-        for (int e = 0; e < 8; e++) {
-            const int c = 8 * g + e;
-            float s = 0.f;
-#pragma unroll
-            for (int tap = 0; tap < 9; tap++) s = fmaf(w[tap * C + c], d[tap], s);
-            r8[e] = f2bf(bf2f(x8[e]) > 0.f ? s : 0.f);
-        }
-        st16(dx + p * C + 8 * g, r);
-    }
-}
-
-hipError_t launch_edge_out_bwd(const float* dy, const float* w, const uint16_t* x, int C,
-                               uint16_t* dx, int B, int H, int W, hipStream_t s) {
-    const long long n = (long long)B * H * W;
-    const dim3 g((unsigned)((n + 255) / 256));
+hipError_t launch_edge_out_grad(const float* dy, const uint16_t* x, int C, const float* w, uint16_t* dx,
+                                float* part, int nblk, int B, int H, int W, hipStream_t s) {
     if (C == 32)
-        hipLaunchKernelGGL(edge_out_bwd_kernel<32>, g, dim3(256), 0, s, dy, w, x, dx, B, H, W);
+        hipLaunchKernelGGL((edge_grad_kernel<32, true>), dim3(nblk), dim3(256), 0, s, dy, x, w, dx, part, B, H, W);
     else if (C == 64)
-        hipLaunchKernelGGL(edge_out_bwd_kernel<64>, g, dim3(256), 0, s, dy, w, x, dx, B, H, W);
-    else
-        return hipErrorInvalidValue;
-    return hipGetLastError();
-}
-
-template <int C>
-__global__ void edge_out_wgrad_kernel(const float* dy, const uint16_t* x, float* part, int B, int H,
-                                      int W) {
-    constexpr int G = C / 8, LANES = 256 / G;
-    __shared__ float red[9 * C + 1];
-    const long long n = (long long)B * H * W;
-    const long long ppb = (n + gridDim.x - 1) / gridDim.x;
-    const long long p0 = blockIdx.x * ppb, p1 = p0 + ppb < n ? p0 + ppb : n;
-    const int t = threadIdx.x, g = t % G;
-    float acc[9][8];
-    float bs = 0.f;
-#pragma unroll
-    for (int k = 0; k < 9; k++)
-#pragma unroll
-        for (int e = 0; e < 8; e++) acc[k][e] = 0.f;
-    for (int i = t; i < 9 * C + 1; i += 256) red[i] = 0.f;
-    for (long long p = p0 + t / G; p < p1; p += LANES) {
-        int bb, yy, xx;
-        pix_coords(p, H, W, bb, yy, xx);
-        const float d = dy[p];
-        if (g == 0) bs += d;
-#pragma unroll
-        for (int tap = 0; tap < 9; tap++) {
-            const int y2 = yy + tap / 3 - 1, x2 = xx + tap % 3 - 1;
-            if (y2 < 0 || y2 >= H || x2 < 0 || x2 >= W) continue;
-            const uint4 v = ld16(x + (((long long)bb * H + y2) * W + x2) * C + 8 * g);
-            const uint16_t* v8 = (const uint16_t*)&v;
-#pragma unroll
-            for (int e = 0; e < 8; e++) acc[tap][e] = fmaf(d, bf2f(v8[e]), acc[tap][e]);
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < 9; k++)
-#pragma unroll
-        for (int e = 0; e < 8; e++) atomicAdd(&red[k * C + 8 * g + e], acc[k][e]);
-    if (g == 0) atomicAdd(&red[9 * C], bs);
-    __syncthreads();
-    for (int i = t; i < 9 * C + 1; i += 256) part[(long long)blockIdx.x * (9 * C + 1) + i] = red[i];
-}
-
-hipError_t launch_edge_out_wgrad(const float* dy, const uint16_t* x, int C, float* part, int nblk,
-                                 int B, int H, int W, hipStream_t s) {
-    if (C == 32)
-        hipLaunchKernelGGL(edge_out_wgrad_kernel<32>, dim3(nblk), dim3(256), 0, s, dy, x, part, B, H, W);
-    else if (C == 64)
-        hipLaunchKernelGGL(edge_out_wgrad_kernel<64>, dim3(nblk), dim3(256), 0, s, dy, x, part, B, H, W);
+        hipLaunchKernelGGL((edge_grad_kernel<64, true>), dim3(nblk), dim3(256), 0, s, dy, x, w, dx, part, B, H, W);
     else
         return hipErrorInvalidValue;
     return hipGetLastError();

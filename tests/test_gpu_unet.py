@@ -212,6 +212,42 @@ def test_network_gradients_match_oracle():
     net.close()
 
 
+@pytest.mark.parametrize("base,B,H,W", [(32, 1, 2, 2), (32, 3, 10, 66), (32, 1, 16, 64), (64, 2, 18, 34), (64, 1, 6, 70)])
+def test_edge_layer_gradients_sizes(base, B, H, W):
+    """Gradients of the first and last layer around the strips of their kernel (64 or 32
+    columns x 8 rows).  The layers between copy their channels (one centre tap) and the
+    numbers are small integers, so every activation is exact in bf16 and no ReLU sits on
+    a rounding: the last layer's gradients are FP32 sums (1e-5), the first layer's
+    terms carry one bf16 rounding of 2^-9 each (2^-7 of the whole)."""
+    print(f"case base={base} {B}x{H}x{W}", flush=True)
+    rng = np.random.default_rng(H * W)
+    layout = {name: (ci, co, w, b) for name, ci, co, w, b in RU.param_layout(base, 2)}
+    net = RU.Unet(base, 2, seed=6)
+    p = np.zeros_like(net.get_params())
+    for name in ("enc0b", "dec0a", "dec0b"):
+        ci, co, w, _ = layout[name]
+        k = p[w:w + 9 * ci * co].reshape(co, 9, ci)
+        first = ci - base                                   # dec0a: the skip's channels come last
+        for c in range(co):
+            k[c, 4, first + c] = 1
+    ci, co, w, b = layout["enc0a_in"]
+    p[w:w + 9 * co] = rng.integers(-2, 3, 9 * co)
+    p[b:b + co] = rng.integers(0, 3, co)
+    ci, co, w, b = layout["out"]
+    p[w:w + 9 * ci] = rng.integers(-1, 2, 9 * ci)
+    net.set_params(p)
+    x = rng.integers(-2, 3, (B, H, W)).astype(np.float32)
+    t = rng.integers(-3, 4, (B, H, W)).astype(np.float32)
+    loss, g = net.loss_grad(torch.from_numpy(x).to(DEV), torch.from_numpy(t).to(DEV), 1.0)
+    rl, rg = U.UnetRef(base, 2).loss_grad(p.astype(np.float64), x, t, 1.0)
+    assert abs(loss - rl) <= 1e-5 * rl
+    for name, tol in (("out", 1e-5), ("enc0a_in", 2.0 ** -7)):
+        ci, co, w, b = layout[name]
+        assert rel(g[w:w + 9 * ci * co], rg[w:w + 9 * ci * co]) <= tol, name
+        assert rel(g[b:b + co], rg[b:b + co]) <= tol, name
+    net.close()
+
+
 def test_training_reduces_loss():
     """Adam on a fixed batch: the network learns a 3x3 blur of its input."""
     net = RU.Unet(32, 4, seed=5)
