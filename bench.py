@@ -430,13 +430,25 @@ def dtype_of(args):
     return "f16" if (args.store != "f32" and args.lds_half) else "f32"
 
 
+def on_matrix_cores(args, S):
+    """Default FP32 plans of whole stacks of 64 (of large images: 2048^2 is)."""
+    return (args.interp == "linear" and args.store == "f32" and args.slices_per_item == 0 and S >= 64
+            and args.tile in (-1, 0))
+
+
 def roofline_of(args, S, achieved, traffic):
-    """FP32 kernels against the FP32 vector peak; the opt-in matrix-core kernel (FP16
+    """FP32 kernels against the FP32 vector peak; stacks of 64 FP32 slices and the opt-in matrix-core kernel (FP16
     rows, --slices-per-item 32) against the dense FP16 MFMA peak.  achieved is
     algorithmic (6 FLOP per update) either way; the MFMA kernel executes 32 FLOP per
     update (16-sample windows), reported beside it."""
     m32 = (args.store != "f32" and args.lds_half and args.slices_per_item == 32 and S >= 32
            and args.interp == "linear")
+    if on_matrix_cores(args, S):
+        # FP32 stacks as products of operands split into two FP16 halves: 8 samples x 2
+        # halves x 2 halves, 64 FLOP per update
+        return {"bound": "mfma", "achieved": round(achieved, 3), "peak": FP16_PEAK_TFLOPS, "unit": "TFLOP/s",
+                "frac": round(achieved / FP16_PEAK_TFLOPS, 4), "traffic": traffic,
+                "mfma_executed": round(achieved * 64 / FLOP_PER_UPDATE, 3)}
     if m32:
         return {"bound": "mfma", "achieved": round(achieved, 3), "peak": FP16_PEAK_TFLOPS, "unit": "TFLOP/s",
                 "frac": round(achieved / FP16_PEAK_TFLOPS, 4), "traffic": traffic,
@@ -461,8 +473,8 @@ def main():
     ap.add_argument("--lds-half", type=int, default=0, help="FP16 pairs in LDS for 16-bit stores")
     ap.add_argument("--persistent", type=int, default=1)
     ap.add_argument("--slices-per-item", type=int, default=0,
-                    help="LINEAR: slices of identical geometry per work item (0 = four with FP32 "
-                         "rows, sixteen with FP16 pairs; or 1, 2, 4, 8, 16, 32)")
+                    help="LINEAR: slices of identical geometry per work item (0 = 64, then four, with "
+                         "FP32 rows, sixteen with FP16 pairs; or 1, 2, 4, 8, 16, 32)")
     ap.add_argument("--graph", type=int, default=1)
     ap.add_argument("--no-cpu", action="store_true", help="skip the CPU baseline leg")
     ap.add_argument("--texture", type=float, default=0.02,
@@ -587,9 +599,9 @@ def main():
     if args.workload == "c2" and args.interp == "linear" and args.store == "f32" and S == 64 \
             and args.proj == 1800 and args.width == 2048 and args.slices_per_item in (0, 2, 4) \
             and args.tile in (-1, 0) and args.chunk == 0:
-        # the FP32 default runs four slices per work item; two per item has its own figure
+        # one figure for each number of slices per work item
         traffic = read_traffic("bp_linear_c2_traffic.md" if args.slices_per_item == 2
-                               else "bp_linear4_c2_traffic.md")
+                               else "bp_x64_c2.md" if on_matrix_cores(args, S) else "bp_linear4_c2_traffic.md")
     config = {"workload": desc, "slices": S, "interp": args.interp, "store": args.store,
               "persistent": bool(args.persistent), "graph": bool(args.graph),
               "lds_half": bool(args.lds_half), "slices_per_item": args.slices_per_item, "updates": updates}
