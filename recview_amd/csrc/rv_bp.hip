@@ -665,8 +665,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 4 : 1) bp_tiled_kernel(BpLa
     }
 }
 
-// BP_LINEAR / BP_LINEAR2 / BP_LINEAR4 on parts of a 64 x 64 tile, for launches whose
-// tiles are too few to fill the chip (bp_sub_parts).  A workgroup owns 16 PX x 16 PY
+// BP_LINEAR / BP_LINEAR2 / BP_LINEAR4 on parts of a tile, for launches whose tiles are too few to fill the chip (bp_sub_parts).  A workgroup owns 16 PX x 16 PY
 // pixels of a tile and forms coordinates and samples as bp_tiled_kernel does on the
 // whole tile (same origin, same operations, same order of the sums), so the images are
 // the same bit for bit.  It stages only the samples its part sees; the rows of the next
@@ -683,19 +682,25 @@ struct SubCfg {
     using T = typename std::conditional<NS == 1, float2, float4>::type;
 };
 
+// The tile: w x h pixels, and the bits of a pixel's offset in it that bp_tiled_kernel
+// covers in steps of 8 i and 8 j (8 (PX - 1), 8 (PY - 1) of its instantiation).
+struct SubTile {
+    int w, h, mx, my;
+};
+
 template <int NS, int PX, int PY>
-__global__ void __launch_bounds__(256) bp_sub_kernel(BpLaunch L)
+__global__ void __launch_bounds__(256) bp_sub_kernel(BpLaunch L, SubTile E)
 {
     using F = SubCfg<NS, PX, PY>;
     using C = typename F::C;
     using T = typename F::T;
     constexpr int SEG = C::SEG, CH = F::CH, NQ = F::NQ;
-    constexpr int NSX = 64 / C::TW, NSUB = NSX * (64 / C::TH);
+    const int nsx = E.w / C::TW, nsub = nsx * (E.h / C::TH);
     __shared__ float4 tab[CH];
     __shared__ T data[CH * NQ * SEG];
 
-    int item = blockIdx.x / NSUB;
-    const int sub = blockIdx.x % NSUB;
+    int item = blockIdx.x / nsub;
+    const int sub = blockIdx.x % nsub;
     if (L.item_order) item = L.item_order[item];
     int lo = 0, hi = L.nslices - 1;
     while (lo < hi) {
@@ -705,17 +710,17 @@ __global__ void __launch_bounds__(256) bp_sub_kernel(BpLaunch L)
     lo = __builtin_amdgcn_readfirstlane(lo);
     const BpSlice& S = L.slices[lo];
     const int t = item - S.tile_base;
-    const int X0 = (t % S.tiles_x) * 64, Y0 = (t / S.tiles_x) * 64;
-    const int sx = (sub % NSX) * C::TW, sy = (sub / NSX) * C::TH;       // the part's place in the tile
+    const int X0 = (t % S.tiles_x) * E.w, Y0 = (t / S.tiles_x) * E.h;
+    const int sx = (sub % nsx) * C::TW, sy = (sub / nsx) * C::TH;       // the part's place in the tile
     const int out_n = S.out_n, nang = S.nang, N = S.row_len;
     if (X0 + sx >= out_n || Y0 + sy >= out_n) return;
 
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int wx = sx + (wave & 1) * C::WX, wy = sy + (wave >> 1) * C::WY;     // the wave's pixels in the tile
-    // bp_tiled_kernel's lane offset (X & 39) and pixel step 8 i (X & 24) of pixel X of the tile
-    const float dxl = (float)((wx & 32) + (lane & 7)), dyl = (float)((wy & 32) + (lane >> 3));
-    const float xi = (float)(wx & 24), yj = (float)(wy & 24);
+    // bp_tiled_kernel's lane offset and pixel steps 8 i, 8 j of the lane's first pixel
+    const float dxl = (float)((wx & ~E.mx) + (lane & 7)), dyl = (float)((wy & ~E.my) + (lane >> 3));
+    const float xi = (float)(wx & E.mx), yj = (float)(wy & E.my);
 
     // staging: one angle of the chunk per thread, samples j0, j0 + TPA, ... of its part
     const int sa = tid / F::TPA, j0 = tid % F::TPA;
@@ -729,8 +734,8 @@ __global__ void __launch_bounds__(256) bp_sub_kernel(BpLaunch L)
     auto fetch_rows = [&](int a0) {
         const bool ok = a0 + sa < nang;
         const double ut = e.u0 + (double)X0 * e.dux + (double)Y0 * e.duy;
-        const double u64 = ut + fmin(0.0, 63 * e.dux) + fmin(0.0, 63 * e.duy);
-        const int s0 = (int)floor(u64) - 1;                                     // the tile's
+        const double utile = ut + fmin(0.0, (E.w - 1) * e.dux) + fmin(0.0, (E.h - 1) * e.duy);
+        const int s0 = (int)floor(utile) - 1;                                    // the tile's
         const double us = ut + sx * e.dux + sy * e.duy + fmin(0.0, (C::TW - 1) * e.dux) +
                           fmin(0.0, (C::TH - 1) * e.duy);
         jlo = max((int)floor(us) - 1 - s0, 0);                                  // the part's, from the tile's
@@ -854,32 +859,47 @@ __global__ void __launch_bounds__(256) bp_sub_kernel(BpLaunch L)
 //   333^2 x 240 (36 tiles)     125 / 43 / 37 / 33     512^2 x 450 (64)    221 / 72 / 60 / 63
 //   700^2 x 500 (121)          238 / 82 / 82 / 107   1024^2 x 900 (256)  418 / 192 / 224 / 289
 //   1536^2 x 1200 (576)        620 / 507 / 552 / 767 2048^2 x 1800 (1024) 1085 / 1244 / 1423 / 1997
+//   1700^2 x 900 (729)         499 / 505
 // Four slices per item: 384^2 x 225 (36 tiles) 236 / 124 / 71 / 62, 384^2 x 225 x 16
 // (144) 249 / 137 / 130 / 132, 800^2 x 600 (169) 621 / 287 / 301 / 313, 1024^2 x 900 x 8
-// (512) 905 / 882 / 1097 / 1213, 2048^2 x 1800 (1024) 2311 / 3393 / 4171 / 4608.
+// (512) 905 / 882 / 1097 / 1213, 2048^2 x 1800 (1024) 2311 / 3393 / 4171 / 4608.  Pairs, whole
+// tiles (64 x 128 and 128 x 64 below 700^2) / parts: 384^2 x 225 270 / 52, 512^2 x 450 505 / 91,
+// 600^2 x 450 506 / 109, 1024^2 x 900 562 / 268, 1400^2 x 1200 (484) 767 / 642.
+// (Tiles counted as 64 x 64 pixels, whatever the tile configuration.)
 int bp_sub_parts(int mode, int tile, int total_items)
 {
-    if (tile != 0) return 0;
-    if (mode == BP_LINEAR) return total_items <= 48 ? 16 : total_items <= 96 ? 8 : total_items <= 768 ? 4 : 0;
-    if (mode == BP_LINEAR2 || mode == BP_LINEAR4)
-        return total_items <= 80 ? 16 : total_items <= 150 ? 8 : total_items <= 512 ? 4 : 0;
+    const long long n = (long long)total_items * bp_tile_side(tile) * bp_tile_h(tile) / 4096;
+    if (mode == BP_LINEAR) return n <= 48 ? 16 : n <= 96 ? 8 : n <= 640 ? 4 : 0;
+    if (mode == BP_LINEAR2 || mode == BP_LINEAR4) return n <= 80 ? 16 : n <= 150 ? 8 : n <= 512 ? 4 : 0;
     return 0;
 }
 
-template <int NS>
-static void launch_sub(const BpLaunch& L, int parts, hipStream_t stream)
+template <int NS, int PX, int PY>
+static void launch_sub(const BpLaunch& L, hipStream_t stream)
 {
-    const dim3 grid(L.total_items * parts);
-    if (parts == 16) hipLaunchKernelGGL((bp_sub_kernel<NS, 1, 1>), grid, dim3(256), 0, stream, L);
-    else if (parts == 8) hipLaunchKernelGGL((bp_sub_kernel<NS, 2, 1>), grid, dim3(256), 0, stream, L);
-    else hipLaunchKernelGGL((bp_sub_kernel<NS, 2, 2>), grid, dim3(256), 0, stream, L);
+    using C = TileCfg<PX, PY>;
+    SubTile E{bp_tile_side(L.tile), bp_tile_h(L.tile), 24, 24};      // <4, 4>
+    if (L.tile == 1) E.my = 56;                                     // <4, 8>
+    if (L.tile == 2) E.mx = E.my = 8;                               // <2, 2>
+    if (L.tile == 3) E.mx = 56;                                     // <8, 4>
+    if (L.tile == 4) E.mx = 8;                                      // <2, 4>
+    const int nsub = (E.w / C::TW) * (E.h / C::TH);
+    hipLaunchKernelGGL((bp_sub_kernel<NS, PX, PY>), dim3(L.total_items * nsub), dim3(256), 0, stream, L, E);
+}
+
+template <int NS>
+static void launch_sub_parts(const BpLaunch& L, int parts, hipStream_t stream)
+{
+    if (parts == 16) launch_sub<NS, 1, 1>(L, stream);
+    else if (parts == 8) launch_sub<NS, 2, 1>(L, stream);
+    else launch_sub<NS, 2, 2>(L, stream);
 }
 
 void launch_bp_sub(const BpLaunch& L, int parts, hipStream_t stream)
 {
-    if (L.mode == BP_LINEAR) launch_sub<1>(L, parts, stream);
-    else if (L.mode == BP_LINEAR2) launch_sub<2>(L, parts, stream);
-    else launch_sub<4>(L, parts, stream);
+    if (L.mode == BP_LINEAR) launch_sub_parts<1>(L, parts, stream);
+    else if (L.mode == BP_LINEAR2) launch_sub_parts<2>(L, parts, stream);
+    else launch_sub_parts<4>(L, parts, stream);
 }
 
 // BpSlice::tgeom: the tile origin of every (tile, angle), formed exactly as

@@ -220,7 +220,7 @@ inline int work_run(int total_items, bool deal)
 }
 
 void launch_bp(const BpLaunch& L, int grid, hipStream_t stream);
-// Parts a 64 x 64 tile is split into over workgroups (launch_bp_sub), for launches of
+// Parts 64 x 64 pixels of a tile are split into over workgroups (launch_bp_sub), for launches of
 // one FP32 slice, pair or four per item whose tiles are too few; 0: whole tiles.
 int bp_sub_parts(int mode, int tile, int total_items);
 void launch_bp_sub(const BpLaunch& L, int parts, hipStream_t stream);

@@ -790,9 +790,10 @@ def test_plan_parts_of_tiles_equal_whole_tiles(W, P, k, store, dtype):
         sinos.append(phantom.to_int16(x) if dtype == "i16" else x)
     fill = [fbp.SliceSpec(1800, np.array([0.0, 90.0], np.float32), 900.3, sino_dtype=dtype) for _ in range(k)]
     rows = [torch.zeros(2, 1800, dtype=sinos[0].dtype) for _ in range(k)]
-    _, few = _run(specs, sinos, store=store)
-    for persistent in (False, True):
-        _, many = _run(specs + fill, sinos + rows, store=store, persistent=persistent)
-        for i in range(k):
-            assert np.array_equal(few[i], many[i]), (i, persistent)
-    assert np.abs(few[0]).max() > 0
+    for tile in range(5):
+        _, few = _run(specs, sinos, store=store, tile=tile)
+        for persistent in (False, True):
+            _, many = _run(specs + fill, sinos + rows, store=store, persistent=persistent, tile=tile)
+            for i in range(k):
+                assert np.array_equal(few[i], many[i]), (i, persistent, tile)
+        assert np.abs(few[0]).max() > 0
