@@ -306,8 +306,10 @@ typedef struct {
                           * larger FP32 images (from 640^2 pixels, 256 projections and 5e8 updates
                           * per slice on, tile 0) on the matrix cores instead (each value as
                           * two FP16 halves, FP32 sums: closer to FP64 than the vector kernels, not bit
-                          * for bit theirs; ask for 4 to have those), sixteen with FP16 pairs (lds_half:
-                          * one FP16 dot product per update and one power-of-two scale per work
+                          * for bit theirs, which a class's leftovers run; ask for 4 to have one
+                          * rounding for all; slices with a sample that is not finite, or with a
+                          * few rows 2^14 above most others, run on the vector kernels too),
+                          * sixteen with FP16 pairs (lds_half: one FP16 dot product per update and one power-of-two scale per work
                           * item; eight on the 64x64 tile, which has no sixteen-slice kernel); or
                           * 1, 2, 4, 8, 16, 32 (at most 4 with FP32 values in LDS; 8 on the 64x64,
                           * 32x32 and 32x64 tiles, 16 on the 32x32 and 32x64 tiles, else fewer;

@@ -9,7 +9,9 @@
 //   W[k][pixel] = max(0, 1 - |u_pixel - j0 - k|).
 //
 // FP32 operands are kept as sums of two FP16 values, p = ph + pl and w = wh + wl
-// (each rounded to nearest: 22 significant bits and the sign of the low part).  The
+// (each rounded to nearest: 22 significant bits and the sign of the low part; samples are
+// scaled by one power of two per slice, so those below 2^-17 of the slice's largest are
+// kept to 2^-40 of that instead).  The
 // 32-long contraction of v_mfma_f32_16x16x32_f16 is two angles x eight samples x
 // {ph, pl}; against it stand wh twice and wl twice, so two products do the whole
 // (ph + pl) (wh + wl) of 2 x 256 updates with FP32 sums and drop nothing.
@@ -18,8 +20,9 @@
 // j + 16 (i / 4), element i % 4.  Lane group g = lane / 16 holds samples 2g and
 // 2g + 1 of the window, as [ph ph pl pl] of the first angle, then of the second.
 //
-// Samples that are not finite would reach every pixel of a window (0 * NaN), so they
-// are packed as zeros and added to the image afterwards (bpx_nonfinite_kernel).
+// Slices that this does not suit -- samples that are not finite, which would reach every
+// pixel of a window (0 * NaN), or a few rows far above all others -- are back-projected
+// again by the vector kernel (bpx_apart_kernel).
 #include "rv_internal.h"
 
 #include <cfloat>
@@ -444,55 +447,69 @@ __global__ void __launch_bounds__(64 * NW, NG == 4 ? 2 : 4) bpx_kernel(BpLaunch 
 }
 
 // ------------------------------------------------------------ packed rows
-// Largest finite magnitude of a slice's filtered rows: block part of slice, by
-// kBpxParts parts.
-__global__ void __launch_bounds__(256) bpx_max_kernel(const PackJob* jobs, float* part)
+// Largest magnitude of every filtered row, infinity where a sample is not finite: one
+// wave per row, rows of slice y of job z.
+__global__ void __launch_bounds__(256) bpx_row_max_kernel(const PackJob* jobs)
 {
     const PackJob& J = jobs[blockIdx.z];
-    const float* rows = (const float*)J.rows[blockIdx.y];
-    const long long n = (long long)J.nrows * J.N;
+    const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (row >= J.nrows) return;
+    const float* src = (const float*)J.rows[blockIdx.y] + (long long)row * J.N;
     float m = 0.f;
-    const long long head = min(n, (long long)((16 - ((uintptr_t)rows & 15)) & 15) / 4), quads = (n - head) / 4;
     auto take = [&](float x) {
         const float v = fabsf(x);
-        if (v <= FLT_MAX) m = fmaxf(m, v);                 // finite values only
+        m = v <= FLT_MAX ? fmaxf(m, v) : INFINITY;
     };
-    const float4* body = (const float4*)(rows + head);
-    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < quads; i += (long long)kBpxParts * 256) {
+    const int head = min(J.N, (int)(((16 - ((uintptr_t)src & 15)) & 15) / 4)), quads = (J.N - head) / 4;
+    const float4* body = (const float4*)(src + head);
+    for (int i = lane; i < quads; i += 64) {
         const float4 v = body[i];
         take(v.x); take(v.y); take(v.z); take(v.w);
     }
     // the values before and after the 16-byte quads (at most six)
-    const long long rest = threadIdx.x < head ? threadIdx.x : threadIdx.x + 4 * quads;
-    if (blockIdx.x == 0 && rest < n) take(rows[rest]);
+    const int rest = lane < head ? lane : lane + 4 * quads;
+    if (rest < J.N) take(src[rest]);
     for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
-    __shared__ float red[4];
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
-    __syncthreads();
-    if (threadIdx.x == 0)
-        part[((size_t)blockIdx.z * BP_MAX_SLICES_PER_ITEM + blockIdx.y) * kBpxParts + blockIdx.x] =
-            fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    if (lane == 0) J.row_max[(size_t)blockIdx.y * J.nrows + row] = m;
 }
 
-// Exponent of each slice: its samples times 2^-e lie within 2^15.
-__global__ void __launch_bounds__(64) bpx_exponent_kernel(const PackJob* jobs, const float* part)
+// Exponent of each slice: its samples times 2^-e lie within 2^15.  A slice runs apart
+// (bpx_apart_kernel) where the matrix products would lose what it holds: when a sample
+// is not finite, and when one of a few rows is so large that most others lie below 2^-14
+// of it, from where on the split would leave them fewer bits than FP32 does (rows at
+// 2^-16 of the largest still keep 23, at 2^-20 they keep 20, at 2^-24 16).  Rows of
+// zeros are exact and do not count.
+__global__ void __launch_bounds__(256) bpx_exponent_kernel(const PackJob* jobs)
 {
     const PackJob& J = jobs[blockIdx.y];
+    const float* row_max = J.row_max + (size_t)blockIdx.x * J.nrows;
+    __shared__ float red[4];
     float m = 0.f;
-    for (int k = threadIdx.x; k < kBpxParts; k += 64)
-        m = fmaxf(m, part[((size_t)blockIdx.y * BP_MAX_SLICES_PER_ITEM + blockIdx.x) * kBpxParts + k]);
+    for (int k = threadIdx.x; k < J.nrows; k += 256) m = fmaxf(m, row_max[k]);
     for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+    __syncthreads();
+    m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    const float low = m * 0x1p-14f;
+    int weak = 0, strong = 0;
+    for (int k0 = 0; k0 < J.nrows; k0 += 256) {
+        const float v = k0 + threadIdx.x < J.nrows ? row_max[k0 + threadIdx.x] : 0.f;
+        weak += __syncthreads_count(v > 0.f && v < low);
+        strong += __syncthreads_count(v >= low && v > 0.f);
+    }
     if (threadIdx.x == 0) {
         int e = 15;
-        if (m > 0.f) frexpf(m, &e);
+        const bool finite = m <= FLT_MAX;
+        if (finite && m > 0.f) frexpf(m, &e);
         ((int*)J.gscale)[blockIdx.x] = e - 15;
+        ((int*)J.gscale)[J.ns + blockIdx.x] = !finite || weak > strong;
     }
 }
 
 // Packed row: [plane 2 q + part][pair][16 slices] of FP16 pairs (samples 2j, 2j + 1),
 // part 0 the high and part 1 the low halves of group q, kBpxPad zero samples on
-// either side; samples that are not finite are zero and mark the row in J.bad.
-// Thread: one slice, eight consecutive samples.
+// either side.  A slice's samples only reach its own sums, so those of slices that run
+// apart may be anything.  Thread: one slice, eight consecutive samples.
 __global__ void __launch_bounds__(256) bpx_pack_kernel(const PackJob* jobs)
 {
     const PackJob& J = jobs[blockIdx.z];
@@ -505,9 +522,6 @@ __global__ void __launch_bounds__(256) bpx_pack_kernel(const PackJob* jobs)
     const float* src = (const float*)J.rows[16 * q + i] + (long long)row * N;
     xuint2* o = (xuint2*)J.out + ((size_t)row * ng + q) * pairs * 16 + i;
     const bool aligned = ((uintptr_t)src & 15) == 0;       // then src + j is, j being a multiple of four
-    __shared__ int bad[16];
-    if (threadIdx.x < 16) bad[threadIdx.x] = 0;
-    __syncthreads();
     for (int p0 = 4 * (threadIdx.x >> 4); p0 < pairs; p0 += 64) {
         const int j0 = 2 * p0 - kBpxPad;
         float v[8];
@@ -520,9 +534,7 @@ __global__ void __launch_bounds__(256) bpx_pack_kernel(const PackJob* jobs)
             for (int k = 0; k < 8; k++) v[k] = (used && j0 + k >= 0 && j0 + k < N) ? src[j0 + k] : 0.f;
         }
 #pragma unroll
-        for (int k = 0; k < 8; k++)
-            if (fabsf(v[k]) <= FLT_MAX) v[k] = ldexpf(v[k], sh);
-            else { v[k] = 0.f; bad[i] = 1; }
+        for (int k = 0; k < 8; k++) v[k] = ldexpf(v[k], sh);
 #pragma unroll
         for (int k = 0; k < 4; k++) {
             if (p0 + k >= pairs) break;
@@ -532,61 +544,49 @@ __global__ void __launch_bounds__(256) bpx_pack_kernel(const PackJob* jobs)
             o[(size_t)(p0 + k) * 16] = xuint2{__builtin_bit_cast(unsigned int, h), __builtin_bit_cast(unsigned int, l)};
         }
     }
-    __syncthreads();
-    if (used && threadIdx.x < 16) J.bad[(size_t)(16 * q + threadIdx.x) * J.nrows + row] = (unsigned char)bad[threadIdx.x];
 }
 
-// Adds what the samples that are not finite contribute: per pixel the interpolated
-// values that are not finite, on the vector kernels' 64 x 64 tiles and with their
-// coordinate.  Block: slice x of item y, part z of the tiles.  Without such rows a block
-// ends after reading their marks (64 x 1800 of them: 6 us in all).
-__global__ void __launch_bounds__(256) bpx_nonfinite_kernel(BpLaunch L)
+// Work list of the slices that run apart, one slice per item on the vector ALU
+// (bp_tiled_kernel, whose images they keep bit for bit): rest holds an entry for every
+// slice of the items, in order; the tiles of those marked fill the end of the list and
+// the persistent launch's counter starts there, so that nothing marked is nothing to do.
+__global__ void __launch_bounds__(1024) bpx_apart_kernel(const BpSlice* items, int nitems, BpSlice* rest, int* order,
+                                                         int total, unsigned int* counter)
 {
-    const BpSlice& S = L.slices[blockIdx.y];
-    const int sl = blockIdx.x, nang = S.nang, N = S.row_len, out_n = S.out_n;
-    const unsigned char* bad = S.bad + (size_t)sl * nang;
-    const float* rows = (const float*)(sl == 0 ? S.rows_0 : S.rows_x[sl - 1]);
-    float* out = (float*)(sl == 0 ? S.out : S.out_x[sl - 1]);
-    __shared__ int list[1024], count;
-    for (int r0 = 0; r0 < nang; r0 += 1024) {
+    constexpr int NS = bp_slices_per_item(BP_LINEAR_X64);
+    __shared__ int marked[NS];
+    const int tid = threadIdx.x;
+    int end = total;
+    for (int q = 0; q < nitems; q++) {
+        const int mark = tid < NS ? ((const int*)items[q].gscale)[NS + tid] : 0;
+        if (tid < NS) marked[tid] = mark;
+        if (!__syncthreads_or(mark)) continue;
+        for (int e = 0; e < NS; e++) {
+            if (!marked[e]) continue;
+            BpSlice& R = rest[NS * q + e];
+            const int n = R.tiles_x * R.tiles_y;
+            end -= n;
+            for (int t = tid; t < n; t += 1024) order[end + t] = R.tile_base + t;
+            if (tid == 0) R.out = e == 0 ? items[q].out : items[q].out_x[e - 1];
+        }
         __syncthreads();
-        if (threadIdx.x == 0) count = 0;
-        __syncthreads();
-        for (int r = r0 + threadIdx.x; r < min(r0 + 1024, nang); r += 256)
-            if (bad[r]) list[atomicAdd(&count, 1)] = r;
-        __syncthreads();
-        if (count == 0) continue;
-        const int n = count;
-        for (int Y = blockIdx.z; Y < out_n; Y += gridDim.z)
-            for (int X = threadIdx.x; X < out_n; X += 256) {
-                float sum = 0.f;
-                for (int k = 0; k < n && sum == sum; k++) {
-                    const AngleEntry& e = S.ang[list[k]];
-                    const double ut = e.u0 + (double)(X & ~63) * e.dux + (double)(Y & ~63) * e.duy;
-                    const int s0 = (int)floor(ut + fmin(0.0, 63.0 * e.dux) + fmin(0.0, 63.0 * e.duy)) - 1;
-                    const float dux = (float)e.dux, duy = (float)e.duy;
-                    const float u = fmaf((float)(X & 24), dux, fmaf((float)(Y & 24), duy,
-                                    fmaf((float)(Y & 39), duy, fmaf((float)(X & 39), dux, (float)(ut - (double)s0)))));
-                    const int q = s0 + (int)u;
-                    if (q < 0 || q >= N) continue;
-                    const float* p = rows + (size_t)list[k] * N + q;
-                    const float d = q == N - 1 ? 0.f : p[1] - p[0];
-                    const float v = fmaf(u, d, p[0] - (float)(q - s0) * d);
-                    if (!(fabsf(v) <= FLT_MAX)) sum += v;
-                }
-                if (sum != 0.f) out[(size_t)Y * out_n + X] += sum * S.out_scale;
-            }
     }
+    if (tid == 0) *counter = end;
 }
 
-void launch_bpx_pack(const PackJob* d_jobs, int njobs, int ns, int max_rows, float* part, hipStream_t stream)
+void launch_bpx_pack(const PackJob* d_jobs, int njobs, int ns, int max_rows, hipStream_t stream)
 {
     if (njobs <= 0 || max_rows <= 0) return;
-    hipLaunchKernelGGL(bpx_max_kernel, dim3(kBpxParts, ns, njobs), dim3(256), 0, stream, d_jobs, part);
-    hipLaunchKernelGGL(bpx_exponent_kernel, dim3(ns, njobs), dim3(64), 0, stream, d_jobs, (const float*)part);
+    hipLaunchKernelGGL(bpx_row_max_kernel, dim3((max_rows + 3) / 4, ns, njobs), dim3(256), 0, stream, d_jobs);
+    hipLaunchKernelGGL(bpx_exponent_kernel, dim3(ns, njobs), dim3(256), 0, stream, d_jobs);
     hipLaunchKernelGGL(bpx_pack_kernel, dim3(bpx_angles(max_rows), ns / 16, njobs), dim3(256), 0, stream, d_jobs);
 }
 
+void launch_bpx_apart(const BpSlice* items, int nitems, BpSlice* rest, int* order, int total, unsigned int* counter,
+                      hipStream_t stream)
+{
+    hipLaunchKernelGGL(bpx_apart_kernel, dim3(1), dim3(1024), 0, stream, items, nitems, rest, order, total, counter);
+}
 
 template <int NG, int NW>
 static void prepare_one()
@@ -609,7 +609,6 @@ static void launch_one(const BpLaunch& L, int grid, hipStream_t stream)
 void launch_bpx(const BpLaunch& L, int grid, hipStream_t stream)
 {
     launch_one<4, 8>(L, grid, stream);
-    hipLaunchKernelGGL(bpx_nonfinite_kernel, dim3(64, L.nslices, 64), dim3(256), 0, stream, L);
 }
 
 }  // namespace rv

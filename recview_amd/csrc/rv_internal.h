@@ -140,7 +140,6 @@ constexpr long long bp_m32_chunks(int N) { return (N + 7) / 8; }
 constexpr int kBpxPad = 48;
 constexpr int bpx_pairs(int N) { return (N + 1) / 2 + kBpxPad; }
 constexpr int bpx_angles(int nang) { return (nang + 3) / 4 * 4; }
-constexpr int kBpxParts = 64;           // partial maxima per slice
 constexpr int kBpxPart = 64 * 32 * 32;  // sums of one work item (a segment's totals)
 
 // Per-angle table entry.  LINEAR: detector coordinate of pixel (ix, iy) of the
@@ -170,15 +169,12 @@ struct BpSlice {
     const void* rows_x[BP_MAX_SLICES_PER_ITEM - 1];   // BP_LINEAR2: rows, scales and image
     const float* scales_x[BP_MAX_SLICES_PER_ITEM - 1]; // of the item's other slices
     void* out_x[BP_MAX_SLICES_PER_ITEM - 1];
-    const float* gscale;    // FP16 multi-slice modes: the item scale (device, set by the pack pass)
+    const float* gscale;    // FP16 multi-slice modes: the item scale (device, set by the pack pass);
+                            // BP_LINEAR_X64: int exponents of the slices, then 1 for those that run apart
     // BP_LINEAR2: per (tile, angle) the tile geometry (dux, duy, ut - s0, s0 as int
     // bits), [tiles][nang], built once per plan, read one angle ahead instead of
     // formed in LDS per chunk; nullptr: formed per chunk
     const float4* tgeom;
-    // BP_LINEAR_X64: filtered rows of the item's first slice (rows_x: the others'), and
-    // [slice][angle] 1 where such a row has a sample that is not finite
-    const void* rows_0;
-    unsigned char* bad;
 };
 
 struct BpLaunch {
@@ -258,8 +254,8 @@ struct PackJob {
     int store;              // 0 f32, 1 f16, 2 bf16
     int nrows, N;           // rows of N samples, row stride N
     void* out;              // [nrows][N] packed samples
-    float* gscale;          // FP16 pairs: the item scale, written by the scale pass
-    unsigned char* bad;     // BP_LINEAR_X64: BpSlice::bad, written by the pack pass
+    float* gscale;          // BpSlice::gscale, written by the scale pass
+    float* row_max;         // BP_LINEAR_X64: [slice][row] largest magnitudes (infinity: not finite)
 };
 // Item scales of FP16-pair jobs (jobs of other kinds are skipped), then the
 // packing of njobs jobs of one kind (0: FP32 pairs; 3: FP32, four slices; 2 / 4 /
@@ -291,13 +287,15 @@ bool bp_deals_runs(int mode);               // persistent work dealt to the XCDs
 int bp_max_chunk(int mode);                 // largest chunk a mode supports
 size_t bp_lds_bytes(int mode, int tile, int chunk);
 // BP_LINEAR_X64: kernel attributes (outside stream captures), tile geometry table of
-// 32 x 32 tiles ([tiles][bpx_angles(nang)]), packing of njobs jobs of ns slices (part:
-// njobs * BP_MAX_SLICES_PER_ITEM * kBpxParts floats) and back-projection.
+// 32 x 32 tiles ([tiles][bpx_angles(nang)]), packing of njobs jobs of ns slices,
+// back-projection, and the work list of the slices that run apart after it.
 void bpx_prepare();
 void launch_bpx_geometry(const AngleEntry* ang, int nang, int tiles_x, int ntiles, int N, float4* out,
                          hipStream_t stream);
-void launch_bpx_pack(const PackJob* d_jobs, int njobs, int ns, int max_rows, float* part, hipStream_t stream);
+void launch_bpx_pack(const PackJob* d_jobs, int njobs, int ns, int max_rows, hipStream_t stream);
 void launch_bpx(const BpLaunch& L, int grid, hipStream_t stream);
+void launch_bpx_apart(const BpSlice* items, int nitems, BpSlice* rest, int* order, int total, unsigned int* counter,
+                      hipStream_t stream);
 void launch_zero_u32(unsigned int* p, int n, hipStream_t stream);
 // Tile geometry table of BpSlice::tgeom for tiles of tw x th pixels, ntiles of them
 // in rows of tiles_x, over nang angle entries.

@@ -74,6 +74,11 @@ struct Group {
     int total_items = 0;
     int grid = 0;
     int parts = 0;               // workgroups per tile (bp_sub_parts), 0: persistent or one per tile
+    // BP_LINEAR_X64: every slice as an item of its own, for those that run apart
+    std::vector<rv::BpSlice> rest;
+    rv::BpSlice* d_rest = nullptr;
+    int* d_rest_order = nullptr;
+    int rest_items = 0, rest_grid = 0, rest_chunk = 0;
 };
 
 }  // namespace
@@ -101,7 +106,6 @@ struct rv_plan_opaque {
     rv::PackJob* d_pack_jobs = nullptr;
     int n_pack = 0;
     bool pack_half = false;
-    float* d_xpart = nullptr;            // BP_LINEAR_X64 packing: partial maxima
     float* d_xsum = nullptr;             // BP_LINEAR_X64: segment totals, per workgroup
     struct PackRange { int first, count, kind, rows; };
     std::vector<PackRange> pack_ranges;  // one per group: jobs of one kind
@@ -129,6 +133,8 @@ void plan_free(rv_plan_t p)
     for (auto& G : p->groups) {
         (void)hipFree(G.d_slices);
         (void)hipFree(G.d_order);
+        (void)hipFree(G.d_rest);
+        (void)hipFree(G.d_rest_order);
     }
     (void)hipFree(p->d_rows);
     (void)hipFree(p->d_scales);
@@ -141,7 +147,6 @@ void plan_free(rv_plan_t p)
     (void)hipFree(p->d_gscale);
     (void)hipFree(p->d_tgeom);
     (void)hipFree(p->d_pack_jobs);
-    (void)hipFree(p->d_xpart);
     (void)hipFree(p->d_xsum);
     (void)hipFree(p->d_fft_work);
     delete p;
@@ -300,7 +305,7 @@ void launch_packing(rv_plan_t p, hipStream_t st)
     if (p->pack_half) rv::launch_pack_scales(p->d_pack_jobs, p->n_pack, st);
     for (const auto& R : p->pack_ranges) {
         if (R.kind >= kPackX)
-            rv::launch_bpx_pack(p->d_pack_jobs + R.first, R.count, R.kind - kPackX, R.rows, p->d_xpart, st);
+            rv::launch_bpx_pack(p->d_pack_jobs + R.first, R.count, R.kind - kPackX, R.rows, st);
         else
             rv::launch_pack(p->d_pack_jobs + R.first, R.count, R.kind, p->store, R.rows, st);
     }
@@ -329,6 +334,16 @@ int launch_backprojection(rv_plan_t p, hipStream_t st, bool pack = true)
             L.counter = ctr;
             L.part = p->d_xsum;
             rv::launch_bpx(L, G.grid, st);
+            rv::launch_bpx_apart(G.d_slices, L.nslices, G.d_rest, G.d_rest_order, G.rest_items, ctr, st);
+            L.slices = G.d_rest;
+            L.nslices = (int)G.rest.size();
+            L.total_items = G.rest_items;
+            L.item_order = G.d_rest_order;
+            L.run = rv::work_run(G.rest_items, false);
+            L.mode = rv::BP_LINEAR;
+            L.tile = 0;
+            L.chunk = G.rest_chunk;
+            rv::launch_bp(L, G.rest_grid, st);
             continue;
         }
         if (G.parts) {
@@ -678,13 +693,16 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
                                          : (size_t)N * packed_size(mode);
     };
     auto packed_rows = [](int mode, int nang) -> size_t { return is_x(mode) ? rv::bpx_angles(nang) : nang; };
+    auto row_max_bytes = [](int nang) -> size_t {          // PackJob::row_max
+        return align_up(sizeof(float) * rv::bp_slices_per_item(rv::BP_LINEAR_X64) * nang, 256);
+    };
     size_t packed_bytes = 0, n_half = 0;
     for (const auto& G : p->groups)
         if (packed_size(G.mode))
             for (int s : G.slices) {
                 packed_bytes += align_up(packed_rows(G.mode, p->sl[s].nang) * packed_row(G.mode, p->sl[s].g.N), 256);
-                if (is_x(G.mode)) packed_bytes += align_up((size_t)64 * p->sl[s].nang, 256);   // BpSlice::bad
-                n_half += is_x(G.mode) ? (size_t)rv::bp_slices_per_item(G.mode)
+                if (is_x(G.mode)) packed_bytes += row_max_bytes(p->sl[s].nang);
+                n_half += is_x(G.mode) ? 2 * (size_t)rv::bp_slices_per_item(G.mode)
                                               : G.mode != rv::BP_LINEAR2 && G.mode != rv::BP_LINEAR4;
             }
     std::vector<rv::PackJob> pack_jobs;
@@ -819,7 +837,7 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
                 J.N = S.g.N;
                 J.out = p->d_packed + packed_off;
                 J.gscale = J.half || x ? p->d_gscale + half_idx : nullptr;
-                half_idx += J.half ? 1 : x ? ns : 0;
+                half_idx += J.half ? 1 : x ? 2 * ns : 0;
                 if (q == 0)
                     p->pack_ranges.push_back(
                         {(int)pack_jobs.size(), 0, x ? kPackX + ns : J.half ? ns : ns == 4 ? 3 : 0, 0});
@@ -833,9 +851,20 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
                 B.gscale = J.gscale;
                 packed_off += align_up(packed_rows(G.mode, S.nang) * packed_row(G.mode, S.g.N), 256);
                 if (x) {
-                    pack_jobs.back().bad = B.bad = p->d_packed + packed_off;
-                    B.rows_0 = J.rows[0];
-                    packed_off += align_up((size_t)64 * S.nang, 256);
+                    pack_jobs.back().row_max = (float*)(p->d_packed + packed_off);
+                    packed_off += row_max_bytes(S.nang);
+                    for (int e = 0; e < ns; e++) {
+                        rv::BpSlice R = B;
+                        R.rows = J.rows[e];
+                        R.row_stride = S.g.N;
+                        R.gscale = nullptr;
+                        R.tgeom = nullptr;
+                        R.tiles_x = (S.out_n + rv::bp_tile_side(0) - 1) / rv::bp_tile_side(0);
+                        R.tiles_y = (S.out_n + rv::bp_tile_h(0) - 1) / rv::bp_tile_h(0);
+                        R.tile_base = G.rest_items;
+                        G.rest_items += R.tiles_x * R.tiles_y;
+                        G.rest.push_back(R);
+                    }
                 }
             }
         }
@@ -849,6 +878,14 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
             rv::bpx_prepare();
             G.grid = std::min(rv::device_cu_count(device), G.total_items);     // one workgroup per CU
             x_grid = std::max(x_grid, G.grid);
+            if (!rv::hip_ok(hipMalloc(&G.d_rest, sizeof(rv::BpSlice) * G.rest.size()), "slice table") ||
+                !rv::hip_ok(hipMalloc(&G.d_rest_order, sizeof(int) * G.rest_items), "work list") ||
+                !rv::hip_ok(hipMemcpy(G.d_rest, G.rest.data(), sizeof(rv::BpSlice) * G.rest.size(),
+                                      hipMemcpyHostToDevice), "slices"))
+                return fail(p, std::string("plan upload failed: ") + RecviewLastMessage());
+            G.rest_chunk = rv::bp_default_chunk(rv::BP_LINEAR, 0);
+            G.rest_grid = std::min(rv::bp_blocks_per_cu_tg(rv::BP_LINEAR, 0, G.rest_chunk, false) *
+                                       rv::device_cu_count(device), G.rest_items);
             continue;
         }
         G.parts = rv::bp_sub_parts(G.mode, G.tile, G.total_items);
@@ -862,12 +899,7 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
     }
     p->cur_out.assign(nslices, nullptr);
     if (!xg_tab.empty()) {
-        size_t n = 0;
-        for (const auto& R : p->pack_ranges)
-            if (R.kind >= kPackX) n = std::max(n, (size_t)R.count);
-        if (!rv::hip_ok(hipMalloc(&p->d_xpart, sizeof(float) * n * rv::BP_MAX_SLICES_PER_ITEM * rv::kBpxParts),
-                        "partial maxima") ||
-            !rv::hip_ok(hipMalloc(&p->d_xsum, sizeof(float) * rv::kBpxPart * x_grid), "segment totals"))
+        if (!rv::hip_ok(hipMalloc(&p->d_xsum, sizeof(float) * rv::kBpxPart * x_grid), "segment totals"))
             return fail(p, std::string("plan allocation failed: ") + RecviewLastMessage());
     }
     if (!pack_jobs.empty()) {

@@ -797,3 +797,51 @@ def test_plan_parts_of_tiles_equal_whole_tiles(W, P, k, store, dtype):
             for i in range(k):
                 assert np.array_equal(few[i], many[i]), (i, persistent, tile)
         assert np.abs(few[0]).max() > 0
+
+
+def test_plan_matrix_core_stack_runs_unsuited_slices_apart():
+    """Slices of a stack on the matrix cores whose samples do not suit the split into
+    FP16 halves -- one not finite, one whose row of angle 0 is far above all others --
+    have the images of one slice per item bit for bit, in a stack at the end of the plan
+    too; the slices beside them are those of a plan without such rows.  The row far above
+    lights the first columns only: beside them the error against FP64 is that of four
+    slices per item."""
+    W, P, S = 640, 1221, 128
+    fdeg, c = phantom.angles_deg(P), W / 2 + 0.37
+    rng = np.random.default_rng(31)
+    # rows that change slowly, as those of four slices per item are summed most exactly
+    base = np.cumsum(rng.normal(size=(P, W)), 1).astype(np.float32)
+    base -= base.mean(1, keepdims=True)
+    rows = [base * np.float32(0.5 + i % 5) for i in range(S)]
+    hot, bad = 5, (70, 127)
+    clean = [r.copy() for r in rows]
+    rows[hot][0] = 0
+    rows[hot][0, :4] = np.abs(rows[hot]).max() * 2.0 ** 26
+    rows[bad[0]][700, 5] = np.nan
+    rows[bad[1]][0, W - 1] = -np.inf
+    specs = [fbp.SliceSpec(W, fdeg, c) for _ in range(S)]
+
+    def images(data, **kw):
+        plan = fbp.FbpPlan(specs, **kw)
+        outs = [torch.full((W, W), 7.0, device="cuda") for _ in range(S)]
+        for i, r in enumerate(data):
+            plan.set_filtered_rows(i, torch.from_numpy(r).cuda())
+        torch.cuda.synchronize()
+        plan.backproject(outs)
+        torch.cuda.synchronize()
+        tile = plan.info(0)["tile_w"]
+        plan.close()
+        return [o.cpu().numpy() for o in outs], tile
+
+    wide, tile = images(rows, persistent=True)
+    assert tile == 32                                                  # the matrix-core items
+    one, _ = images(rows, slices_per_item=1)
+    four, _ = images(rows, slices_per_item=4, persistent=True)
+    plain, _ = images(clean)
+    for i in (hot,) + bad:
+        assert np.array_equal(wide[i], one[i], equal_nan=True), i
+    for i in set(range(S)) - {hot, *bad}:
+        assert np.array_equal(wide[i], plain[i]), i
+    ref = O.bp_rows_linear_f64(rows[hot], fdeg, O.geometry(W, 2, c))[:, 16:]
+    err = [float(np.sqrt(np.mean((x[hot][:, 16:] - ref) ** 2))) for x in (wide, four)]
+    assert err[0] <= 1.1 * err[1], err
