@@ -10,7 +10,8 @@ OUT = os.path.join(HERE, "librecview_hip.so")
 HARNESS = os.path.join(HERE, "recview_harness")
 
 HOST_SOURCES = ["rv_common.cpp", "rv_compat.cpp", "rv_plan.cpp", "rv_offset.cpp", "rv_unet.cpp", "rv_output.cpp"]
-DEVICE_SOURCES = ["rv_filter.hip", "rv_bp.hip", "rv_bpx.hip", "rv_stitch.hip", "rv_unet.hip", "rv_sinogram.hip", "rv_output.hip"]
+DEVICE_SOURCES = ["rv_filter.hip", "rv_bp.hip", "rv_bpsub.hip", "rv_bpx.hip", "rv_stitch.hip", "rv_unet.hip",
+                  "rv_sinogram.hip", "rv_output.hip"]
 
 # -ffp-contract=off: the parity modes reproduce the reference's FP32 operation
 # order; FMAs are written explicitly where they are wanted.  Packed FP32
