@@ -575,8 +575,9 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
         for (int s = 0; s < nslices; s++) classes.push_back({s});
     }
 
-    // RECVIEW_GEOMETRY_TABLES=0 (diagnostics, tests): every group forms its geometry
-    // per chunk, as when the tables would exceed the budget
+    // RECVIEW_GEOMETRY_TABLES=0 (diagnostics, tests): groups whose kernel can form its
+    // geometry per chunk do so, as when the tables would exceed the budget.  The matrix-core
+    // stacks have no other source of theirs: the switch leaves kernels and images as they are.
     const char* tg_env = std::getenv("RECVIEW_GEOMETRY_TABLES");
     const bool tg_allowed = !(tg_env && tg_env[0] == '0');
     const size_t tg_budget = (size_t)8 << 30;
@@ -595,7 +596,7 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
             // FP32 stacks on the matrix cores (default plans only: an explicit
             // slices_per_item keeps the vector kernels and their rounding)
             int kx = 0;
-            if (p->mode == rv::BP_LINEAR && p->store == 0 && opt->slices_per_item == 0 && tg_allowed && left >= 64 &&
+            if (p->mode == rv::BP_LINEAR && p->store == 0 && opt->slices_per_item == 0 && left >= 64 &&
                 tile == 0 && x64_pays(p->sl[cls[i]].out_n, p->sl[cls[i]].nang)) {
                 const int c = (int)(&cls - classes.data());
                 const SliceState& S = p->sl[cls[i]];

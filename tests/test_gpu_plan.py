@@ -845,3 +845,18 @@ def test_plan_matrix_core_stack_runs_unsuited_slices_apart():
     ref = O.bp_rows_linear_f64(rows[hot], fdeg, O.geometry(W, 2, c))[:, 16:]
     err = [float(np.sqrt(np.mean((x[hot][:, 16:] - ref) ** 2))) for x in (wide, four)]
     assert err[0] <= 1.1 * err[1], err
+
+
+def test_plan_geometry_switch_keeps_matrix_core_stacks(monkeypatch):
+    """The diagnostic switch that has geometry formed per chunk changes no image of a
+    stack on the matrix cores and its leftover slice either."""
+    W, P, S = 640, 1221, 65
+    base, fdeg, c = _sino(W, P, 88, photons=1e4)
+    sinos = [torch.from_numpy(base) * (0.5 + 0.01 * i) for i in range(S)]
+    specs = [fbp.SliceSpec(W, fdeg, c) for _ in range(S)]
+    _, tables = _run(specs, sinos, persistent=True)
+    monkeypatch.setenv("RECVIEW_GEOMETRY_TABLES", "0")
+    plan, per_chunk = _run(specs, sinos, persistent=True)
+    assert plan.info(0)["tile_w"] == 32
+    for i in range(S):
+        assert np.array_equal(per_chunk[i], tables[i]), i
