@@ -720,13 +720,21 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
     // 8192^2 x 3600 needs 3.8 GiB), groups beyond that form theirs per chunk.
     // A table depends on the geometry and the tile configuration: the matrix-core
     // grouping moves its slices to 32x32 tiles after the classes are formed, so a
-    // class can run on two tile configurations.
+    // class can run on two tile configurations.  Launches on parts of tiles form theirs
+    // as they go.
     std::vector<int> cls_of(nslices, -1);
     for (size_t c = 0; c < classes.size(); c++)
         for (int s : classes[c]) cls_of[s] = (int)c;
     std::map<std::pair<int, int>, std::pair<size_t, int>> tg_tab;   // (class, tile) -> (offset, slice)
     for (auto& G : p->groups) {
-        if (!tg_allowed || !rv::bp_has_tgeom(G.mode)) continue;
+        int base = 0;
+        for (int s : G.slices) {
+            p->sl[s].tile_base = base;
+            base += p->sl[s].tiles_x * p->sl[s].tiles_y;
+        }
+        G.total_items = base;
+        if (!is_x(G.mode)) G.parts = rv::bp_sub_parts(G.mode, G.tile, G.total_items);
+        if (!tg_allowed || G.parts || !rv::bp_has_tgeom(G.mode)) continue;
         G.tgeom = true;
         for (int s : G.slices) {
             const int c = cls_of[s];
@@ -767,14 +775,8 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
         // slice order inside the group: longest projection lists first
         std::vector<int> ord = G.slices;
         std::stable_sort(ord.begin(), ord.end(), [&](int a, int b) { return p->sl[a].nang > p->sl[b].nang; });
-        int base = 0;
-        for (int s : G.slices) {
-            p->sl[s].tile_base = base;
-            base += p->sl[s].tiles_x * p->sl[s].tiles_y;
-        }
-        G.total_items = base;
         std::vector<int> order;
-        order.reserve(base);
+        order.reserve(G.total_items);
         for (int s : ord) {
             const SliceState& S = p->sl[s];
             if (is_x(G.mode)) {
@@ -889,7 +891,7 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
                                        rv::device_cu_count(device), G.rest_items);
             continue;
         }
-        G.parts = rv::bp_sub_parts(G.mode, G.tile, G.total_items);
+        if (G.parts) continue;
         (void)rv::bp_blocks_per_cu_tg(G.mode, G.tile, G.chunk, G.tgeom);     // sets LDS attributes outside capture
         if (opt->persistent) {
             const int per_cu = rv::bp_blocks_per_cu_tg(G.mode, G.tile, G.chunk, G.tgeom);

@@ -860,3 +860,21 @@ def test_plan_geometry_switch_keeps_matrix_core_stacks(monkeypatch):
     assert plan.info(0)["tile_w"] == 32
     for i in range(S):
         assert np.array_equal(per_chunk[i], tables[i]), i
+
+
+def test_plan_of_few_tiles_holds_no_geometry_tables(monkeypatch):
+    """Launches on parts of tiles read no geometry table (28 MB for this pair), so
+    their plans take the memory of plans without."""
+    specs = [fbp.SliceSpec(1400, phantom.angles_deg(3600), 700.3) for _ in range(2)]
+
+    def held():
+        before = torch.cuda.mem_get_info()[0]
+        plan = fbp.FbpPlan(specs)
+        n = before - torch.cuda.mem_get_info()[0]
+        plan.close()
+        return n
+
+    held()                                             # twiddles, code objects
+    tables = held()
+    monkeypatch.setenv("RECVIEW_GEOMETRY_TABLES", "0")
+    assert abs(tables - held()) < 8 << 20
