@@ -125,7 +125,7 @@ static size_t part_floats(const Unet* u, int B, int H, int W) {
             const int ns = wgrad_splits(L.cin, L.cout, B, h, w);
             m = std::max<size_t>(m, (size_t)ns * (9ull * L.cin * L.cout + L.cout));
         } else {
-            m = std::max<size_t>(m, (size_t)edge_blocks(B, H, W) * (10ull * u->base + 1));
+            m = std::max<size_t>(m, (size_t)edge_blocks(u->C(0), B, H, W) * (10ull * u->base + 1));
         }
     }
     return m;
@@ -306,7 +306,7 @@ static bool forward(Unet* u, const float* in, float scale, hipStream_t s, bool m
 static bool backward(Unet* u, hipStream_t s) {
     const int Lv = u->levels;
     const int B = u->B, H = u->H, W = u->W;
-    const int nb = edge_blocks(B, H, W);
+    const int nb = edge_blocks(u->C(0), B, H, W);
     const ULayer& Lo = u->layers[u->li_out()];
     if (!ok(launch_edge_out_grad(u->dy, u->d[0], u->C(0), u->P + Lo.w, u->g_d[0], u->part, nb, B, H, W, s),
             "edge grad") ||

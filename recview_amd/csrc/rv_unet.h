@@ -67,7 +67,7 @@ hipError_t launch_pack_conv_weights(const float* w, int Cin, int Cout, int trans
 hipError_t launch_edge_in(const float* x, const float* w, const float* b, int C, uint16_t* out,
                           int out_stride, int out_off, int B, int H, int W, hipStream_t s);
 // Its weight gradient: part[blk] = weights [c][tap] (9*C) then biases (C).
-int edge_blocks(int B, int H, int W);
+int edge_blocks(int C, int B, int H, int W);
 hipError_t launch_edge_in_wgrad(const uint16_t* dy, int C, const float* x, float* part, int nblk,
                                 int B, int H, int W, hipStream_t s);
 // Last layer: y[p] = xres[p] + b + sum W[tap][c] * X[p + d(tap)][c]  (C -> 1, fp32 out).

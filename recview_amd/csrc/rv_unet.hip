@@ -838,11 +838,6 @@ hipError_t launch_edge_in(const float* x, const float* w, const float* b, int C,
     return hipGetLastError();
 }
 
-int edge_blocks(int B, int H, int W) {
-    const long long n = (long long)B * H * W;
-    return (int)std::max(1LL, std::min(1024LL, (n + 4095) / 4096));
-}
-
 // Gradients of the two edge layers, whose one side is an image v (the input, or dy of the
 // output layer) and whose other side is activations c of C channels: every pixel's C
 // channels against the 3 x 3 neighbours in v,
@@ -856,6 +851,15 @@ int edge_blocks(int B, int H, int W) {
 // 16 x 512^2 x 32: last layer 350 us (each activation read for nine taps) and 240 us for
 // dX apart -> 227 us in one; first layer 196 -> 92 us.
 constexpr int kEdgeRows = 8;
+
+// A workgroup per strip, up to 1024, which fill the chip and bound the parts (one per
+// 4096 pixels, 8 for 2 x 128^2, left most of it idle: that whole gradient took 1290 us, with
+// 64 workgroups 1200; 4 x 256^2 1700 and 1600).
+int edge_blocks(int C, int B, int H, int W) {
+    const int lanes = 256 / (C / 8);
+    const long long strips = (long long)B * ((H + kEdgeRows - 1) / kEdgeRows) * ((W + lanes - 1) / lanes);
+    return (int)std::max(1LL, std::min(1024LL, strips));
+}
 
 template <int C, bool OUT>
 __global__ __launch_bounds__(256) void edge_grad_kernel(const float* v, const uint16_t* c, const float* w,
