@@ -887,7 +887,9 @@ __global__ __launch_bounds__(256) void edge_grad_kernel(const float* v, const ui
 #pragma unroll
             for (int k = 0; k < 3; k++) {
                 const int xx = x + k - 1;
-                r[k] = (y >= 0 && y < H && xx >= 0 && xx < W) ? v[img + (long long)y * W + xx] : 0.f;
+                // nothing past the image, whose zero activations would make NaN of an infinity
+                const bool in = y >= 0 && y < H && xx >= 0 && xx < W && x < W;
+                r[k] = in ? v[img + (long long)y * W + xx] : 0.f;
             }
         };
         auto load_c = [&](int y) {

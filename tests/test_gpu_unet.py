@@ -283,3 +283,23 @@ def test_trained_network_restores_sparse_view():
     assert s["psnr_phantom"]["restored"] > s["psnr_phantom"]["sparse"] + 1.0
     assert s["ssim_vs_full"]["restored"] > s["ssim_vs_full"]["sparse"]
     net.close()
+
+
+@pytest.mark.parametrize("W", [64, 70])
+def test_edge_layer_gradients_of_an_infinite_target(W):
+    """A target that is infinite in the last column reaches the last layer's weights of
+    the taps that see that pixel from inside the image, and no others, also where the
+    kernel's strips of 64 columns end past the image."""
+    B, H = 1, 12
+    rng = np.random.default_rng(W)
+    net = RU.Unet(32, 2, seed=8)
+    x = torch.from_numpy(rng.standard_normal((B, H, W)).astype(np.float32)).to(DEV)
+    t = torch.zeros_like(x)
+    t[0, 5, W - 1] = float("inf")
+    _, g = net.loss_grad(x, t, 1.0)
+    net.close()
+    layout = {name: (ci, co, w, b) for name, ci, co, w, b in RU.param_layout(32, 2)}
+    ci, co, w, b = layout["out"]
+    taps = np.isfinite(g[w:w + 9 * ci].reshape(3, 3, ci))
+    assert taps[:, 2].all()                            # the neighbour to the right is outside
+    assert not taps[:, :2].all()
