@@ -445,9 +445,9 @@ void CudaReconstResourceFree(RECONST_INFO* ri, bool bCudaDeviceReset)
     CudaReconstMemFree(ri);
     if (bCudaDeviceReset) {
         (void)hipDeviceSynchronize();
+        rv::free_output_works(ri->iStartSino);
         (void)hipDeviceReset();
         rv::drop_device_caches(ri->iStartSino);
-        rv::drop_output_work(ri->iStartSino);
         std::lock_guard<std::mutex> lk(g_deconv_mu);
         g_deconv_work.erase(ri->iStartSino);                       // memory gone with the reset
     }

@@ -99,7 +99,7 @@ bool sinogram_jobs(const SinoWalk& w, std::vector<SinoJob>& jobs);
 // maxima (values of the image type); (min, max) are written to range.
 void launch_output_stage_parts(const void* img, int is_float, int N, int irad2, uint16_t* out, void* part,
                                void* range, hipStream_t s);
-void drop_output_work(int dev);
+void free_output_works(int dev);
 constexpr int kOutputParts = 1024;
 // Squared mask radius of gazoDoc.cpp:4008-4010: r = zoom * center / binning,
 // min(r, N - r) truncated, for the zoom and binning of iInterpolation.

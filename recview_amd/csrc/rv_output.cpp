@@ -49,8 +49,8 @@ std::string tif_text(const char* s, const char* dflt)
 // What a call of RecviewOutputStage works in: the partial minima and maxima on the
 // device, and the (min, max) result in pinned host memory that the GPU writes.  Calls
 // end with their stream's synchronisation, so a work is taken for one call, whatever
-// its thread and stream, and kept for later ones: at most eight of them, dropped with
-// their device (2048^2 floats: 44.7 us a call with an allocation, a copy back, a free and
+// its thread and stream, and kept for later ones: at most eight of them, given back before
+// their device is reset (2048^2 floats: 44.7 us a call with an allocation, a copy back, a free and
 // three launches, 29.9 us now).
 struct OutputWork {
     int dev;
@@ -103,11 +103,16 @@ void give_output_work(const OutputWork& w)
 
 namespace rv {
 
-// after a reset of the device, whose memory is gone
-void drop_output_work(int dev)
+// before a reset of the device, with the device current: the reset takes the device memory
+// and need not take the pinned host memory
+void free_output_works(int dev)
 {
     std::lock_guard<std::mutex> lk(g_work_mu);
-    for (auto it = g_work.begin(); it != g_work.end();) it = it->dev == dev ? g_work.erase(it) : it + 1;
+    for (auto it = g_work.begin(); it != g_work.end();) {
+        if (it->dev != dev) { ++it; continue; }
+        free_output_work(*it);
+        it = g_work.erase(it);
+    }
 }
 
 }  // namespace rv
