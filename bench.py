@@ -430,25 +430,34 @@ def dtype_of(args):
     return "f16" if (args.store != "f32" and args.lds_half) else "f32"
 
 
-def on_matrix_cores(args, S):
-    """Default FP32 plans of whole stacks of 64 (of large images: 2048^2 is)."""
-    return (args.interp == "linear" and args.store == "f32" and args.slices_per_item == 0 and S >= 64
-            and args.tile in (-1, 0))
+def matrix_core_share(plan, specs, shapes, args):
+    """Share of the updates whose slices a default FP32 plan back-projects on the matrix
+    cores: it moves those, and only those, from 64 x 64 tiles to 32 x 32."""
+    if args.interp != "linear" or args.store != "f32":
+        return 0.0
+    on = total = 0.0
+    for s, (spec, (n, p)) in enumerate(zip(specs, shapes)):
+        asked = spec.tile if spec.tile >= 0 else max(args.tile, 0)
+        total += float(n * n * p)
+        if asked == 0 and plan.info(s)["tile_w"] == 32:
+            on += float(n * n * p)
+    return on / total
 
 
-def roofline_of(args, S, achieved, traffic):
-    """FP32 kernels against the FP32 vector peak; stacks of 64 FP32 slices and the opt-in matrix-core kernel (FP16
+def roofline_of(args, S, achieved, traffic, matrix_share):
+    """FP32 kernels against the FP32 vector peak; plans most of whose updates run on the
+    matrix cores as FP32 stacks, and the opt-in matrix-core kernel (FP16
     rows, --slices-per-item 32) against the dense FP16 MFMA peak.  achieved is
     algorithmic (6 FLOP per update) either way; the MFMA kernel executes 32 FLOP per
     update (16-sample windows), reported beside it."""
     m32 = (args.store != "f32" and args.lds_half and args.slices_per_item == 32 and S >= 32
            and args.interp == "linear")
-    if on_matrix_cores(args, S):
+    if matrix_share > 0.5:
         # FP32 stacks as products of operands split into two FP16 halves: 8 samples x 2
-        # halves x 2 halves, 64 FLOP per update
+        # halves x 2 halves, 64 FLOP per update of the slices that run so
         return {"bound": "mfma", "achieved": round(achieved, 3), "peak": FP16_PEAK_TFLOPS, "unit": "TFLOP/s",
                 "frac": round(achieved / FP16_PEAK_TFLOPS, 4), "traffic": traffic,
-                "mfma_executed": round(achieved * 64 / FLOP_PER_UPDATE, 3)}
+                "mfma_executed": round(achieved * matrix_share * 64 / FLOP_PER_UPDATE, 3)}
     if m32:
         return {"bound": "mfma", "achieved": round(achieved, 3), "peak": FP16_PEAK_TFLOPS, "unit": "TFLOP/s",
                 "frac": round(achieved / FP16_PEAK_TFLOPS, 4), "traffic": traffic,
@@ -595,13 +604,14 @@ def main():
                          f"partial-image sum), tau {secs / (N * N * P) * 1e9:.4f} ns; host: {model}{clock}, "
                          f"{threads} threads of {usable} usable, ISA flags {' '.join(flags) or 'none'}"}
 
+    matrix_share = matrix_core_share(plan, specs, shapes, args)
     traffic = None
     if args.workload == "c2" and args.interp == "linear" and args.store == "f32" and S == 64 \
             and args.proj == 1800 and args.width == 2048 and args.slices_per_item in (0, 2, 4) \
             and args.tile in (-1, 0) and args.chunk == 0:
         # one figure for each number of slices per work item
         traffic = read_traffic("bp_linear_c2_traffic.md" if args.slices_per_item == 2
-                               else "bp_x64_c2.md" if on_matrix_cores(args, S) else "bp_linear4_c2_traffic.md")
+                               else "bp_x64_c2.md" if matrix_share > 0.5 else "bp_linear4_c2_traffic.md")
     config = {"workload": desc, "slices": S, "interp": args.interp, "store": args.store,
               "persistent": bool(args.persistent), "graph": bool(args.graph),
               "lds_half": bool(args.lds_half), "slices_per_item": args.slices_per_item, "updates": updates}
@@ -629,7 +639,7 @@ def main():
         "bp_ms": round(bp_ms, 3),
         "config": config,
         "d2h_inclusive": d2h,
-        "roofline": roofline_of(args, S, achieved, traffic),
+        "roofline": roofline_of(args, S, achieved, traffic, matrix_share),
         "cpu_baseline": cpu,
     }
     print(json.dumps(result), flush=True)
