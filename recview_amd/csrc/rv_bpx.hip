@@ -2,8 +2,9 @@
 //
 // Slices of one geometry share every interpolation weight, so for one angle and
 // one 4 x 4-pixel block the linear interpolation of 16 slices is a matrix product
-// over a window of eight detector samples j0 .. j0 + 7 (a block spans at most
-// 3 (|cos| + |sin|) <= 4.25 samples; j0 is even):
+// over a window of eight detector samples j0 .. j0 + 7 (pixels are at most a sample apart,
+// pix_zoom >= 1 in every plan, so a block spans at most 3 (|cos| + |sin|) <= 4.25 samples;
+// j0 is even):
 //
 //   D[slice][pixel] += sum_k P[slice][k] * W[k][pixel],
 //   W[k][pixel] = max(0, 1 - |u_pixel - j0 - k|).
@@ -44,15 +45,17 @@ typedef const __attribute__((address_space(1))) float* gfloat;
 
 namespace bpx {
 constexpr int kTile = 32;                  // pixels per tile side: 8 x 8 blocks
-constexpr int kSeg = 48;                   // staged samples per angle
+constexpr int kSeg = 48;                   // staged samples per angle: a tile spans at most 31 sqrt 2 = 43.9
 constexpr int kPairs = kSeg / 2;
 constexpr int kMaxJ0 = kSeg - 8;           // last window start
 constexpr int kAng = 4;                    // angles per chunk (one contraction)
+constexpr int kWaves = 8;                  // waves of a workgroup
+constexpr int kGroups = bp_slices_per_item(BP_LINEAR_X64) / 16;     // groups of 16 slices
 constexpr int kPlane = kPairs * 128 + 16;  // LDS bytes of one plane (16 slices); the 16 keeps reads of
                                            // different planes from pairing into ds_read2 (whose results
                                            // would need moves into place)
 // three chunks of rows, eight waves' tables of row ends, the work item
-constexpr int lds_bytes(int ng) { return 3 * kAng * ng * kPlane + 8 * 8 * 16 + 16; }
+constexpr int kLdsBytes = 3 * kAng * kGroups * kPlane + kWaves * 8 * 16 + 16;
 }  // namespace bpx
 
 // Tile geometry entry of (tile, angle): cos, sin, the tile origin's coordinate
@@ -116,15 +119,16 @@ __device__ __forceinline__ void static_for(F&& f)
     }
 }
 
-// One work item: NG groups of 16 slices of one 32 x 32 tile, by NW waves of 64 / NW
-// blocks each.
-template <int NG, int NW>
+// One work item: kGroups groups of 16 slices of one 32 x 32 tile, by kWaves waves of a row
+// of eight blocks each.
 __device__ __forceinline__ void bpx_item(const BpSlice& S, int t, float minus_one, xfloat4* part)
 {
     using namespace bpx;
     extern __shared__ xuint4 lds16[];
     unsigned char* lds = (unsigned char*)lds16;
+    constexpr int NG = kGroups, NW = kWaves;
     constexpr int NB = 64 / NW, NSET = NB / 4;         // blocks per wave, in sets of four
+    static_assert(NB == 8, "a wave's blocks are a row of the tile");
     constexpr int ABYTES = NG * kPlane;                // one staged angle
     constexpr int CBYTES = kAng * ABYTES;              // one chunk
     const int N = S.row_len;
@@ -140,8 +144,8 @@ __device__ __forceinline__ void bpx_item(const BpSlice& S, int t, float minus_on
     const float xl = (float)(n & 3), yl = (float)(n >> 2), gneg = -2.f * (float)g;
     // table lane: angle (lane % 16) / 4 of the chunk, block lane % 4 of the wave
     const int ta = (lane >> 2) & 3;
-    const int wx0 = NB == 8 ? 0 : 16 * (wave & 1), wy0 = 4 * (NB == 8 ? wave : wave >> 1);
-    const float bx = (float)(wx0 + 4 * (lane & 3)), by = (float)wy0;
+    const int wy0 = 4 * wave;
+    const float bx = (float)(4 * (lane & 3)), by = (float)wy0;
 
     const int X0 = (t % S.tiles_x) * kTile, Y0 = (t / S.tiles_x) * kTile;
     const int ox = X0 & 32, oy = Y0 & 32;              // offset inside the 64 x 64 tile
@@ -221,8 +225,9 @@ __device__ __forceinline__ void bpx_item(const BpSlice& S, int t, float minus_on
     const int lane8 = 8 * lane;
 
     // Weights of block b for angles 2p and 2p + 1: W(k) of the lane's samples 2g and
-    // 2g + 1, in seven pieces of two to four vector instructions: they end a slot before the
+    // 2g + 1, in kWeights pieces of two to four vector instructions: they end a slot before the
     // products that read them.
+    constexpr int kWeights = 7;
     struct Weights {
         float r[2], t[2], w[2][2];
         xhalf2 h[2], l[2];
@@ -240,7 +245,7 @@ __device__ __forceinline__ void bpx_item(const BpSlice& S, int t, float minus_on
                     // vector kernels' coordinate on their 64 x 64 tile (bp_tiled_kernel)
                     const int j0 = (k.adr[z] - k.buf - ta * ABYTES) / 64;
                     const float last = (float)(N - 1 - (k.sw & ~1) - j0);  // last sample, from the window's start
-                    const float dxl = (float)(ox + 4 * (b & 1) + (n & 3)), xi = (float)((wx0 + 4 * b) & 24);
+                    const float dxl = (float)(ox + 4 * (b & 1) + (n & 3)), xi = (float)((4 * b) & 24);
                     const float dyl = (float)(oy + wy0 % 8 + (n >> 2)), yj = (float)(wy0 & 24);
                     static_for<0, 2>([&](auto ai) {
                         constexpr int a = decltype(ai)::value, A = 2 * p + a, e = 4 * A + b % 4;
@@ -291,7 +296,7 @@ __device__ __forceinline__ void bpx_item(const BpSlice& S, int t, float minus_on
     constexpr int SLOTS = 2 * NG, NSLOT = 2 * NB * SLOTS;      // slots of a step and of a chunk
     constexpr int ST0 = NSLOT / 2 - 2 * SLOTS - PER, BAR = NSLOT / 2, FE0 = BAR + 1, WI0 = BAR + PER + 2;
     constexpr int WID = (NSLOT - SLOTS - WI0) / kWin;          // slots between the window's pieces
-    static_assert(ST0 >= 0 && WID >= 1, "the parts of a chunk fit its slots");
+    static_assert(ST0 >= 0 && WID >= 1 && kWeights < SLOTS, "the parts fit their slots");
     int c0 = 0, c1 = nch;                                  // chunks of the segment
     auto at = [&](int c) { return min(c, c1 - 1); };       // chunks past the last repeat it, unused
     auto rows_at = [&](int c) { return packed + (size_t)at(c) * kAng * row_stride; };
@@ -324,7 +329,7 @@ __device__ __forceinline__ void bpx_item(const BpSlice& S, int t, float minus_on
         xhalf8 Wh[2], Wl[2];
         {
             Weights f;
-            static_for<0, 8>([&](auto i) { weights(i, Int<0>{}, Int<0>{}, win, f, Wh[0], Wl[0]); });
+            static_for<0, kWeights>([&](auto i) { weights(i, Int<0>{}, Int<0>{}, win, f, Wh[0], Wl[0]); });
             const int v0 = address(Int<0>{}, Int<0>{}, Int<0>{}, win), v1 = address(Int<0>{}, Int<0>{}, Int<1>{}, win);
     #pragma unroll
             for (int q = 0; q < NG; q++) {
@@ -350,8 +355,7 @@ __device__ __forceinline__ void bpx_item(const BpSlice& S, int t, float minus_on
                     A = __builtin_amdgcn_mfma_f32_16x16x32_f16(P, (i & 1) ? Wl[p] : Wh[p], A, 0, 0, 0);
                     if constexpr (i < 2) va[i] = address(Int<nb>{}, Int<1 - p>{}, Int<i>{}, k);
                     sample(va[i & 1], q, i & 1, pv[1 - p][q]);
-                    static_for<i * 8 / SLOTS, (i + 1) * 8 / SLOTS>(
-                        [&](auto pc) { weights(pc, Int<nb>{}, Int<1 - p>{}, k, f, Wh[1 - p], Wl[1 - p]); });
+                    if constexpr (i < kWeights) weights(si, Int<nb>{}, Int<1 - p>{}, k, f, Wh[1 - p], Wl[1 - p]);
                     if constexpr (slot >= ST0 && slot < ST0 + PER) stage(Int<slot - ST0>{}, nbuf);
                     if constexpr (slot == BAR) {
                         // the rows were written 2 SLOTS reads ago and more: all but the last
@@ -381,7 +385,7 @@ __device__ __forceinline__ void bpx_item(const BpSlice& S, int t, float minus_on
     }
 
     // lane l, element e of group q: slice 16 q + 4 (l / 16) + e of pixel l % 16
-    const int X = X0 + wx0 + (n & 3);
+    const int X = X0 + (n & 3);
     const int Y = Y0 + wy0 + (n >> 2);
     const int out_n = S.out_n;
     const int* ex = (const int*)S.gscale;
@@ -407,12 +411,11 @@ __device__ __forceinline__ void bpx_item(const BpSlice& S, int t, float minus_on
 // SIMD alone and 26 here.  Slower when tried: products of 32 or 16 slices (weights shared
 // by fewer updates), four angles per contraction with three products (half the LDS reads, but
 // 16-byte reads of four rows each), a second body without the row-end test.
-template <int NG, int NW>
-__global__ void __launch_bounds__(64 * NW, NG == 4 ? 2 : 4) bpx_kernel(BpLaunch L, float minus_one)
+__global__ void __launch_bounds__(64 * bpx::kWaves, 2) bpx_kernel(BpLaunch L, float minus_one)
 {
     extern __shared__ xuint4 lds16[];
-    xfloat4* part = (xfloat4*)L.part + (size_t)blockIdx.x * (16 * NG * bpx::kTile * bpx::kTile / 4);
-    int* item_sh = (int*)((unsigned char*)lds16 + bpx::lds_bytes(NG) - 16);
+    xfloat4* part = (xfloat4*)L.part + (size_t)blockIdx.x * (kBpxPart / 4);
+    int* item_sh = (int*)((unsigned char*)lds16 + bpx::kLdsBytes - 16);
     // the list in eight contiguous parts, one per XCD; a workgroup whose own part is
     // taken goes on with the next
     const int per_xcd = (L.total_items + kXcds - 1) / kXcds;
@@ -442,7 +445,7 @@ __global__ void __launch_bounds__(64 * NW, NG == 4 ? 2 : 4) bpx_kernel(BpLaunch 
         }
         lo = __builtin_amdgcn_readfirstlane(lo);
         const BpSlice& S = L.slices[lo];
-        bpx_item<NG, NW>(S, item - S.tile_base, minus_one, part);
+        bpx_item(S, item - S.tile_base, minus_one, part);
     }
 }
 
@@ -513,14 +516,14 @@ __global__ void __launch_bounds__(256) bpx_exponent_kernel(const PackJob* jobs)
 __global__ void __launch_bounds__(256) bpx_pack_kernel(const PackJob* jobs)
 {
     const PackJob& J = jobs[blockIdx.z];
-    const int N = J.N, pairs = bpx_pairs(N), ng = J.ns / 16;
+    const int N = J.N, pairs = bpx_pairs(N);
     const int row = blockIdx.x;
     if (row >= bpx_angles(J.nrows)) return;
     const bool used = row < J.nrows;               // rows up to a whole chunk are zero
     const int i = threadIdx.x & 15, q = blockIdx.y;
     const int sh = -((const int*)J.gscale)[16 * q + i];
     const float* src = (const float*)J.rows[16 * q + i] + (long long)row * N;
-    xuint2* o = (xuint2*)J.out + ((size_t)row * ng + q) * pairs * 16 + i;
+    xuint2* o = (xuint2*)J.out + ((size_t)row * bpx::kGroups + q) * pairs * 16 + i;
     const bool aligned = ((uintptr_t)src & 15) == 0;       // then src + j is, j being a multiple of four
     for (int p0 = 4 * (threadIdx.x >> 4); p0 < pairs; p0 += 64) {
         const int j0 = 2 * p0 - kBpxPad;
@@ -574,12 +577,13 @@ __global__ void __launch_bounds__(1024) bpx_apart_kernel(const BpSlice* items, i
     if (tid == 0) *counter = end;
 }
 
-void launch_bpx_pack(const PackJob* d_jobs, int njobs, int ns, int max_rows, hipStream_t stream)
+void launch_bpx_pack(const PackJob* d_jobs, int njobs, int max_rows, hipStream_t stream)
 {
+    constexpr int ns = bp_slices_per_item(BP_LINEAR_X64);
     if (njobs <= 0 || max_rows <= 0) return;
     hipLaunchKernelGGL(bpx_row_max_kernel, dim3((max_rows + 3) / 4, ns, njobs), dim3(256), 0, stream, d_jobs);
     hipLaunchKernelGGL(bpx_exponent_kernel, dim3(ns, njobs), dim3(256), 0, stream, d_jobs);
-    hipLaunchKernelGGL(bpx_pack_kernel, dim3(bpx_angles(max_rows), ns / 16, njobs), dim3(256), 0, stream, d_jobs);
+    hipLaunchKernelGGL(bpx_pack_kernel, dim3(bpx_angles(max_rows), bpx::kGroups, njobs), dim3(256), 0, stream, d_jobs);
 }
 
 void launch_bpx_apart(const BpSlice* items, int nitems, BpSlice* rest, int* order, int total, unsigned int* counter,
@@ -588,27 +592,14 @@ void launch_bpx_apart(const BpSlice* items, int nitems, BpSlice* rest, int* orde
     hipLaunchKernelGGL(bpx_apart_kernel, dim3(1), dim3(1024), 0, stream, items, nitems, rest, order, total, counter);
 }
 
-template <int NG, int NW>
-static void prepare_one()
-{
-    (void)hipFuncSetAttribute((const void*)&bpx_kernel<NG, NW>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)bpx::lds_bytes(NG));
-}
-
 void bpx_prepare()
 {
-    prepare_one<4, 8>();
-}
-
-template <int NG, int NW>
-static void launch_one(const BpLaunch& L, int grid, hipStream_t stream)
-{
-    hipLaunchKernelGGL((bpx_kernel<NG, NW>), dim3(grid), dim3(64 * NW), bpx::lds_bytes(NG), stream, L, -1.f);
+    (void)hipFuncSetAttribute((const void*)&bpx_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bpx::kLdsBytes);
 }
 
 void launch_bpx(const BpLaunch& L, int grid, hipStream_t stream)
 {
-    launch_one<4, 8>(L, grid, stream);
+    hipLaunchKernelGGL(bpx_kernel, dim3(grid), dim3(64 * bpx::kWaves), bpx::kLdsBytes, stream, L, -1.f);
 }
 
 }  // namespace rv

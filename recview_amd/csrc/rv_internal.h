@@ -140,7 +140,7 @@ constexpr long long bp_m32_chunks(int N) { return (N + 7) / 8; }
 constexpr int kBpxPad = 48;
 constexpr int bpx_pairs(int N) { return (N + 1) / 2 + kBpxPad; }
 constexpr int bpx_angles(int nang) { return (nang + 3) / 4 * 4; }
-constexpr int kBpxPart = 64 * 32 * 32;  // sums of one work item (a segment's totals)
+constexpr int kBpxPart = bp_slices_per_item(BP_LINEAR_X64) * 32 * 32;   // sums of one work item (a segment's totals)
 
 // Per-angle table entry.  LINEAR: detector coordinate of pixel (ix, iy) of the
 // output grid is u = u0 + ix*dux + iy*duy (all double).  LUT16: the reference
@@ -287,12 +287,12 @@ bool bp_deals_runs(int mode);               // persistent work dealt to the XCDs
 int bp_max_chunk(int mode);                 // largest chunk a mode supports
 size_t bp_lds_bytes(int mode, int tile, int chunk);
 // BP_LINEAR_X64: kernel attributes (outside stream captures), tile geometry table of
-// 32 x 32 tiles ([tiles][bpx_angles(nang)]), packing of njobs jobs of ns slices,
+// 32 x 32 tiles ([tiles][bpx_angles(nang)]), packing of njobs jobs,
 // back-projection, and the work list of the slices that run apart after it.
 void bpx_prepare();
 void launch_bpx_geometry(const AngleEntry* ang, int nang, int tiles_x, int ntiles, int N, float4* out,
                          hipStream_t stream);
-void launch_bpx_pack(const PackJob* d_jobs, int njobs, int ns, int max_rows, hipStream_t stream);
+void launch_bpx_pack(const PackJob* d_jobs, int njobs, int max_rows, hipStream_t stream);
 void launch_bpx(const BpLaunch& L, int grid, hipStream_t stream);
 void launch_bpx_apart(const BpSlice* items, int nitems, BpSlice* rest, int* order, int total, unsigned int* counter,
                       hipStream_t stream);

@@ -60,7 +60,8 @@ struct SliceState {
     size_t pair_off = 0;         // first entry in the pair table
 };
 
-constexpr int kPackX = 100;      // PackRange::kind of BP_LINEAR_X64 jobs: kPackX + slices
+// PackRange::kind of BP_LINEAR_X64 jobs, beside launch_pack's kinds
+constexpr int kPackX = rv::bp_slices_per_item(rv::BP_LINEAR_X64);
 
 struct Group {
     int tile = 0, chunk = 0;
@@ -304,8 +305,8 @@ void launch_packing(rv_plan_t p, hipStream_t st)
 {
     if (p->pack_half) rv::launch_pack_scales(p->d_pack_jobs, p->n_pack, st);
     for (const auto& R : p->pack_ranges) {
-        if (R.kind >= kPackX)
-            rv::launch_bpx_pack(p->d_pack_jobs + R.first, R.count, R.kind - kPackX, R.rows, st);
+        if (R.kind == kPackX)
+            rv::launch_bpx_pack(p->d_pack_jobs + R.first, R.count, R.rows, st);
         else
             rv::launch_pack(p->d_pack_jobs + R.first, R.count, R.kind, p->store, R.rows, st);
     }
@@ -596,7 +597,7 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
             // FP32 stacks on the matrix cores (default plans only: an explicit
             // slices_per_item keeps the vector kernels and their rounding)
             int kx = 0;
-            if (p->mode == rv::BP_LINEAR && p->store == 0 && opt->slices_per_item == 0 && left >= 64 &&
+            if (p->mode == rv::BP_LINEAR && p->store == 0 && opt->slices_per_item == 0 && left >= kPackX &&
                 tile == 0 && x64_pays(p->sl[cls[i]].out_n, p->sl[cls[i]].nang)) {
                 const int c = (int)(&cls - classes.data());
                 const SliceState& S = p->sl[cls[i]];
@@ -607,7 +608,7 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
                         xg_tab[c] = std::make_pair(tg_total, cls[i]);
                         tg_total += bytes;
                     }
-                    kx = 64;
+                    kx = kPackX;
                 }
             }
             const int k = kx ? kx
@@ -843,7 +844,7 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
                 half_idx += J.half ? 1 : x ? 2 * ns : 0;
                 if (q == 0)
                     p->pack_ranges.push_back(
-                        {(int)pack_jobs.size(), 0, x ? kPackX + ns : J.half ? ns : ns == 4 ? 3 : 0, 0});
+                        {(int)pack_jobs.size(), 0, x ? kPackX : J.half ? ns : ns == 4 ? 3 : 0, 0});
                 auto& R = p->pack_ranges.back();
                 R.count++;
                 R.rows = std::max(R.rows, S.nang);
