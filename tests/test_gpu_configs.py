@@ -226,3 +226,28 @@ def test_c4_precision_report():
         os.makedirs(out_dir, exist_ok=True)
         with open(os.path.join(out_dir, "c4_precision.json"), "w") as f:
             json.dump(report, f, indent=1)
+
+
+@pytest.mark.parametrize("spi,tile_w", [(0, 32), (4, 64)])
+def test_c2_fp32_stack_forms(spi, tile_w):
+    """A 64-slice stack of the C2 shape in both forms of FP32 items, 64 slices on the matrix
+    cores (the default) and four on the vector ALU: slices against FP64 filtering + FP64
+    linear back-projection on sampled rows, RMS <= 2e-6 of the range."""
+    import bench
+    W, P, S = 2048, 1800, 64
+    sinos, fdeg, c_det = bench.make_stack(S, P, W, 1002, torch.device("cuda"))
+    g = O.geometry(W, 2, c_det)
+    filt = O.set_filter(g.ndim, 0)
+    rows = np.linspace(0.1 * W, 0.9 * W, 5).astype(int)
+    ys, xs = np.meshgrid(rows, np.arange(W), indexing="ij")
+    inside = ((xs - W / 2) ** 2 + (ys - W / 2) ** 2) <= (0.45 * W) ** 2
+    specs = [fbp.SliceSpec(W, fdeg, c_det) for _ in range(S)]
+    plan, outs = _run(specs, list(sinos), slices_per_item=spi, persistent=True)
+    assert plan.info(0)["tile_w"] == tile_w
+    plan.close()
+    for i in (0, 21, 63):
+        px64 = O.filter_rows_f64(sinos[i].cpu().numpy(), g, filt)
+        ref = O.bp_points_linear_f64(px64, fdeg, g, xs[inside], ys[inside])
+        rms, mx = _errors(outs[i].cpu().numpy()[ys[inside], xs[inside]], ref)
+        print(f"C2 stack slices_per_item={spi} slice {i}: rms {rms:.2e} max {mx:.2e} of range", flush=True)
+        assert rms <= 2e-6, (i, rms, mx)

@@ -878,3 +878,120 @@ def test_plan_of_few_tiles_holds_no_geometry_tables(monkeypatch):
     tables = held()
     monkeypatch.setenv("RECVIEW_GEOMETRY_TABLES", "0")
     assert abs(tables - held()) < 8 << 20
+
+
+def test_plan_matrix_core_stack_of_many_angles():
+    """More than 2048 angles are summed in three segments, the middle one reading and
+    rewriting the totals: within FP32 rounding of four slices per item (2e-5 of the range
+    at any pixel: 1/8 of an FP32 step per projection) and no further from FP64."""
+    W, P, S = 640, 2053, 64
+    base, fdeg, c = _sino(W, P, 41, photons=1e4)
+    sinos = [torch.from_numpy(base).roll(i % 5, 1) * (0.3 + 0.02 * i) for i in range(S)]
+    specs = [fbp.SliceSpec(W, fdeg, c) for _ in range(S)]
+    plan, wide = _run(specs, sinos, persistent=True)
+    assert plan.info(0)["tile_w"] == 32
+    _, four = _run(specs, sinos, slices_per_item=4, persistent=True)
+    g, m = O.geometry(W, 2, c), _circle(W, 0.4)
+    for i in range(S):
+        rng = float(four[i].max() - four[i].min())
+        assert np.abs(wide[i].astype(np.float64) - four[i]).max() <= 2e-5 * rng, i
+    for i in (0, S - 1):
+        ref = O.recon_of64(sinos[i].numpy(), fdeg, g, O.set_filter(g.ndim, 0))
+        rms, _ = _errors(wide[i], ref, m)
+        rms4, _ = _errors(four[i], ref, m)
+        assert rms <= 2e-6 and rms <= 1.1 * rms4, (i, rms, rms4)
+
+
+def test_plan_matrix_core_stacks_of_mixed_geometry():
+    """Two stacks of different width and angle count in one launch, normalised, a
+    sample of the second not finite, with a slice left over: every image as in a plan of its
+    stack alone, eager, and as a graph replayed with another list of images and other rows
+    in between."""
+    shapes, S = ((701, 1018), (640, 1221)), (64, 65)
+    specs, sinos = [], []
+    for (W, P), n in zip(shapes, S):
+        base, fdeg, c = _sino(W, P, 60 + W, photons=1e4)
+        for i in range(n):
+            specs.append(fbp.SliceSpec(W, fdeg, c))
+            sinos.append(torch.from_numpy(base) * (0.5 + 0.01 * i))
+    sinos[64 + 7][300, 9] = float("nan")
+    dev = [x.cuda() for x in sinos]
+    other = [x * 0.5 for x in dev]
+    kw = dict(normalize=True, persistent=True)
+    want = _run(specs[:64], sinos[:64], **kw)[1] + _run(specs[64:], sinos[64:], **kw)[1]
+    plan, got = _run(specs, sinos, **kw)
+    assert plan.info(0)["tile_w"] == plan.info(64)["tile_w"] == 32 and plan.info(128)["tile_w"] == 64
+    half = _run(specs, [x * 0.5 for x in sinos], **kw)[1]
+
+    def same(outs, ref, what):
+        torch.cuda.synchronize()
+        for i, (a, b) in enumerate(zip(outs, ref)):
+            a = a.cpu().numpy() if torch.is_tensor(a) else a
+            assert np.array_equal(a, b, equal_nan=True), (what, i)
+
+    same(got, want, "eager")
+    outs, outs2 = ([torch.zeros(s.W, s.W, device="cuda") for s in specs] for _ in range(2))
+    for rep in range(3):
+        plan.execute(dev, outs, graph=True)
+        same(outs, want, f"graph {rep}")
+        plan.execute(other, outs2)                     # eager, other images
+        same(outs2, half, f"eager between {rep}")
+        same(outs, want, f"graph {rep}, kept")
+    plan.execute(other, outs2, graph=True)             # captured again
+    same(outs2, half, "second graph")
+    plan.close()
+
+
+def test_plan_matrix_core_stack_of_offset_scans_and_shared_rows():
+    """Stacks whose rows are stitched from 360-degree scans, and stacks on the filtered rows
+    of one slice, on the matrix cores: within FP32 rounding of four slices per item (2e-5
+    of the range at any pixel), a shared slice's images all the same."""
+    W, P, S = 400, 901, 64
+    fdeg = (np.arange(2 * P + 1) * (180.0 / P)).astype(np.float32)
+    c = W / 2 + 113.37
+    ell = phantom.random_ellipses(97, count=8)
+    base = phantom.sinogram(ell, W, fdeg, c, scale=0.9 * (2 * (W - c) + W)).float()
+    sinos = [base * (0.5 + 0.01 * i) for i in range(S)]
+    stacks = [([fbp.SliceSpec(W, fdeg, c, offset_ct=True) for _ in range(S)], sinos, 2 * W)]
+    W2, P2 = 701, 1018
+    row, fdeg2, c2 = _sino(W2, P2, 98, photons=1e4)
+    stacks.append(([fbp.SliceSpec(W2, fdeg2, c2, rows_from=0 if i else -1) for i in range(S)],
+                   [torch.from_numpy(row)] * S, W2))
+    for specs, data, N in stacks:
+        plan, wide = _run(specs, data, persistent=True)
+        assert plan.info(0)["tile_w"] == 32 and plan.out_n(0) == N
+        _, four = _run(specs, data, slices_per_item=4, persistent=True)
+        for i in range(S):
+            rng = float(four[i].max() - four[i].min())
+            assert np.abs(wide[i].astype(np.float64) - four[i]).max() <= 2e-5 * rng, (N, i)
+    for i in range(1, S):
+        assert np.array_equal(wide[i], wide[0]), i
+
+
+def test_plan_parts_of_tiles_mixed_sizes_and_shared_rows():
+    """Parts of tiles in launches of several sizes and angle counts, of slices on another
+    slice's rows, and of 16-bit rows' leftover pairs: bit for bit the images of whole tiles
+    (beside slices that fill the launch)."""
+    lone, rows = [], []
+    for i, (W, P) in enumerate(((90, 33), (333, 70), (64, 1), (257, 48))):
+        base, fdeg, c = _sino(W, P, 4400 + i)
+        lone.append(fbp.SliceSpec(W, fdeg, c))
+        rows.append(torch.from_numpy(base))
+    base, fdeg, c = _sino(200, 40, 4410)
+    for j, d in enumerate((0.0, 0.5, -3.25)):
+        lone.append(fbp.SliceSpec(200, fdeg, c + d, rows_from=4 if j else -1))
+        rows.append(torch.from_numpy(base))
+    pair = [fbp.SliceSpec(300, *_sino(300, 50, 4420)[1:]) for _ in range(2)]
+    data = [torch.from_numpy(_sino(300, 50, 4420 + i)[0]) for i in range(2)]
+
+    def fill(n):
+        return ([fbp.SliceSpec(1800, np.array([0.0, 90.0], np.float32), 900.3) for _ in range(n)],
+                [torch.zeros(2, 1800) for _ in range(n)])
+
+    for specs, sinos, n, kw in ((lone, rows, 1, {}), (pair, data, 2, dict(store="f16", lds_half=True))):
+        _, few = _run(specs, sinos, **kw)
+        f, z = fill(n)
+        _, many = _run(specs + f, sinos + z, **kw)
+        for i in range(len(specs)):
+            assert np.abs(few[i]).max() > 0
+            assert np.array_equal(few[i], many[i]), (n, i)
