@@ -324,8 +324,10 @@ typedef struct rv_plan_opaque* rv_plan_t;
 
 /* Builds a plan for nslices slices on device `device`: geometry, filter
  * tables, angle tables, filtered-sinogram workspace, the packed rows of
- * multi-slice work items (FP32: 16 B per sample and slice pair; FP16 pairs:
- * 4 B per sample and slice) and the tile work list.
+ * multi-slice work items (FP32: 16 B per sample and slice pair; FP16 pairs and
+ * the 64-slice FP32 items: 4 B per sample and slice), the geometry tables of
+ * multi-slice FP32 items (16 B per tile and projection, at most 8 GiB), 256 KiB
+ * per compute unit for the sums of 64-slice items, and the tile work list.
  * Returns 0 or a negative error (message in RecviewLastMessage). */
 int rvPlanCreate(rv_plan_t* plan, int device, const RvSliceSpec* specs, int nslices,
                  const RvOptions* opt);
@@ -426,8 +428,8 @@ int RecviewOutputStage(const void* d_img, int is_float, int N, double center, in
  * kernels and results, asynchronous on `stream`: the (min, max) pair is written
  * to the caller's device buffer d_range (two values of the image type) instead
  * of being copied to the host.  The per-block partial minima and maxima live in
- * a library-held 8 KiB device array per GPU (held until the process ends), so
- * calls that overlap on one GPU race; the partials are capped at 1024, which
+ * a library-held 4 KiB device array per GPU (held until the process ends), so
+ * calls that overlap on one GPU race; the partials are capped at 512, which
  * serves every image side up to the limit N <= 65536 (larger N: error). */
 #define RV_OUTPUT_NOALLOC_MAX_SIDE 65536
 int RecviewOutputStageNoAlloc(const void* d_img, int is_float, int N, double center, int iInterpolation,

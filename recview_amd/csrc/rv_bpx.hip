@@ -408,8 +408,8 @@ __device__ __forceinline__ void bpx_item(const BpSlice& S, int t, float minus_on
 // 64 slices of 2048^2 x 1800: 29.5 ms, 1.64e13 updates/s (four slices per item on the
 // vector ALU: 36.5 ms).  Bound by instruction issue: a slot of one product (16 clocks of
 // its pipe), one 8-byte LDS read and three vector instructions takes 24.9 clocks per
-// SIMD alone and 26 here.  Slower when tried: products of 32 or 16 slices (weights shared
-// by fewer updates), four angles per contraction with three products (half the LDS reads, but
+// SIMD alone and 26 here.  Slower than this form when tried: items of 32 or 16 slices (weights
+// shared by fewer updates; not compared with four per item), four angles per contraction with three products (half the LDS reads, but
 // 16-byte reads of four rows each), a second body without the row-end test.
 __global__ void __launch_bounds__(64 * bpx::kWaves, 2) bpx_kernel(BpLaunch L, float minus_one)
 {

@@ -95,12 +95,12 @@ bool sinogram_jobs(const SinoWalk& w, std::vector<SinoJob>& jobs);
 
 // ------------------------------------------------------- output stage
 // Min/max + normalisation to 0..65534 inside the circle of squared radius
-// irad2 (gazoDoc.cpp:3993-4021).  part: room for 1024 partial minima and 1024 partial
-// maxima (values of the image type); (min, max) are written to range.
+// irad2 (gazoDoc.cpp:3993-4021).  part: room for kOutputParts partial minima and as many
+// partial maxima (values of the image type); (min, max) are written to range.
 void launch_output_stage_parts(const void* img, int is_float, int N, int irad2, uint16_t* out, void* part,
                                void* range, hipStream_t s);
 void free_output_works(int dev);
-constexpr int kOutputParts = 1024;
+constexpr int kOutputParts = 512;
 // Squared mask radius of gazoDoc.cpp:4008-4010: r = zoom * center / binning,
 // min(r, N - r) truncated, for the zoom and binning of iInterpolation.
 inline int output_irad2(int N, double center, int iInterpolation)
@@ -118,8 +118,8 @@ inline int output_irad2(int N, double center, int iInterpolation)
 // BP_LINEAR_H2 / H4 / H8 / H16: BP_LINEAR_H over two / four / eight / sixteen;
 // BP_LINEAR_M32: 32 FP16 slices per work item, the updates done as matrix
 // products on the MFMA units (the others in BpSlice::rows_x / scales_x / out_x);
-// BP_LINEAR_X64: 64 FP32 slices per work item as matrix
-// products of operands split into two FP16 halves.
+// BP_LINEAR_X64: 64 FP32 slices per work item as matrix products of operands split into
+// two FP16 halves.
 enum BpMode {
     BP_LINEAR = 0, BP_LUT_F32 = 1, BP_LUT_I32 = 2, BP_LINEAR_H = 3, BP_LINEAR2 = 4,
     BP_LINEAR_H2 = 5, BP_LINEAR_H4 = 6, BP_LINEAR_H8 = 7, BP_LINEAR_H16 = 8, BP_LINEAR_M32 = 9,
@@ -216,8 +216,8 @@ inline int work_run(int total_items, bool deal)
 }
 
 void launch_bp(const BpLaunch& L, int grid, hipStream_t stream);
-// Parts 64 x 64 pixels of a tile are split into over workgroups (launch_bp_sub), for launches of
-// one FP32 slice, pair or four per item whose tiles are too few; 0: whole tiles.
+// Workgroups that share 64 x 64 pixels of a tile (launch_bp_sub), for launches of one FP32
+// slice, pair or four per item whose tiles are too few; 0: whole tiles.
 int bp_sub_parts(int mode, int tile, int total_items);
 void launch_bp_sub(const BpLaunch& L, int parts, hipStream_t stream);
 

@@ -75,7 +75,7 @@ __global__ void __launch_bounds__(256) minmax_kernel(const T* img, long long n, 
     }
 }
 
-// Every workgroup reduces the nparts partial minima / maxima itself (8 KB at most, from
+// Every workgroup reduces the nparts partial minima / maxima itself (4 KB at most, from
 // L2) instead of waiting for a launch that does; the first one writes them to range
 // (max bumped by one unit when equal to the min, gazoDoc.cpp:3999).  Threads take four
 // pixels of a row at a time; vec: rows are 16-byte (image) and 8-byte (out) aligned.
@@ -129,8 +129,7 @@ static void run(const T* img, int N, int irad2, uint16_t* out, T* part, T* range
 {
     const long long n = (long long)N * N;
     // eight 16-byte loads per thread, two workgroups per CU at most
-    const int nparts = (int)std::min<long long>(512, (n + 8191) / 8192);
-    static_assert(512 <= kOutputParts, "the scratch holds the partials");
+    const int nparts = (int)std::min<long long>(kOutputParts, (n + 8191) / 8192);
     T* pmin = part;
     T* pmax = part + kOutputParts;
     const int vec = N % 4 == 0 && ((uintptr_t)img & 15) == 0 && ((uintptr_t)out & 7) == 0;
@@ -153,8 +152,8 @@ void launch_output_stage_parts(const void* img, int is_float, int N, int irad2, 
 
 // ------------------------------------------------ allocation-free output stage
 // The partial minima and maxima of RecviewOutputStageNoAlloc live in this
-// array: 1024 + 1024 four-byte values (8 KiB) on every GPU the library runs on,
-// held until the process ends.  The partials are capped at 1024 whatever the
+// array: 512 + 512 four-byte values (4 KiB) on every GPU the library runs on,
+// held until the process ends.  The partials are capped at 512 whatever the
 // image side, so the array serves every image the entry point accepts.  Host
 // code never passes the array's name to a kernel: it passes the device address
 // hipGetSymbolAddress returns for the current device, kept per device.
@@ -197,8 +196,8 @@ extern "C" int RecviewOutputStageNoAlloc(const void* d_img, int is_float, int N,
     }
     void* part = scratch_on_current_device();
     if (!part) return -1;
-    // every partial the final reduction reads is written by the first launch of
-    // this call, so nothing needs clearing
+    // every partial the second launch reads is written by the first, so nothing needs
+    // clearing
     rv::launch_output_stage_parts(d_img, is_float, N, rv::output_irad2(N, center, iInterpolation), d_out,
                                   part, d_range, (hipStream_t)stream);
     return rv::hip_ok(hipGetLastError(), "output stage") ? 0 : -1;

@@ -32,7 +32,11 @@ constexpr bool is_x(int mode) { return mode == rv::BP_LINEAR_X64; }
 // beside the angles.  Measured for 64 slices, whole execution, four per item against
 // 64 per item (ms): 2048^2 x 1800 38.3 / 31.1, 1024^2 x 900 5.07 / 4.38, 700^2 x 700
 // 2.12 / 1.89, 640^2 x 225 0.68 / 0.68, 2048^2 x 60 1.53 / 1.60, 512^2 x 450 0.81 /
-// 0.83; 70 slices of 800^2 x 300 1.49 / 1.63 (the six slices left over run apart).
+// 0.83; 70 slices of 800^2 x 300 1.49 / 1.63 (the six slices left over are launches of
+// their own).  The line at 5e8 updates keeps clear of those leftovers and with them leaves
+// out a size or two that gain a little (700^2 x 700).  On its near side, 64 slices and with
+// three left over: 640^2 x 1221 3.27 / 3.10 and 4.83 / 3.53, 1448^2 x 256 2.97 / 2.85 and
+// 3.28 / 3.17, 2048^2 x 256 with three 6.11 / 5.58.
 bool x64_pays(int out_n, int nang)
 {
     return out_n >= 640 && nang >= 256 && (double)out_n * out_n * nang >= 5e8;
@@ -532,8 +536,9 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
         return fail(p, "slices_per_item must be 0, 1, 2, 4, 8, 16 or 32");
     // default: sixty-four FP32 slices per item on the matrix cores where x64_pays, else
     // four FP32 slices or sixteen FP16-pair slices per item on the vector ALU (packed
-    // rows; sixteen form on the 32x64 and 32x32 tiles, eight on 64x64).  Measured per 2048^2 x 1800 slice (64-slice stack): FP32 0.57 ms with
-    // four per item, 0.58 ms with two; FP16 pairs 0.367 / 0.381 / 0.492 ms with
+    // rows; sixteen form on the 32x64 and 32x32 tiles, eight on 64x64).  Measured per
+    // 2048^2 x 1800 slice (64-slice stack): FP32 0.46 ms with 64 per item, 0.57 ms with
+    // four, 0.58 ms with two; FP16 pairs 0.367 / 0.381 / 0.492 ms with
     // sixteen (32x64) / eight (64x64) / four per item.  A class's leftovers run as
     // a pair and a single.  32 per item (opt-in) runs the matrix-core kernel: 0.343 ms.
     const int max_per_item = (p->mode == rv::BP_LINEAR_H) ? 32 : 4;
@@ -680,9 +685,10 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
         !rv::hip_ok(hipMemcpy(p->d_ang, ha.data(), sizeof(rv::AngleEntry) * nang_total, hipMemcpyHostToDevice), "angles"))
         return fail(p, std::string("plan upload failed: ") + RecviewLastMessage());
 
-    // packed rows of the multi-slice work items: FP32 pairs 16 B, FP16 pairs 8 / 16 /
-    // 32 / 64 B per sample (two / four / eight / sixteen slices); 32 FP16 slices in
-    // chunks of eight samples
+    // packed rows of the multi-slice work items: FP32 pairs 16 B, fours 32 B, FP16 pairs 8 /
+    // 16 / 32 / 64 B per sample (two / four / eight / sixteen slices); 32 FP16 slices in
+    // chunks of eight samples; 64 FP32 slices 256 B per sample, with zero samples around the
+    // rows and rows up to a whole chunk of angles, and the rows' largest magnitudes
     auto packed_size = [](int mode) -> size_t {
         return is_x(mode) ? 4 * (size_t)rv::bp_slices_per_item(mode)
              : mode == rv::BP_LINEAR_M32 ? 64 : mode == rv::BP_LINEAR_H16 ? 64 : mode == rv::BP_LINEAR_H8 ? 32
