@@ -111,7 +111,7 @@ struct rv_plan_opaque {
     rv::PackJob* d_pack_jobs = nullptr;
     int n_pack = 0;
     bool pack_half = false;
-    float* d_xsum = nullptr;             // BP_LINEAR_X64: segment totals, per workgroup
+    float* d_xsum = nullptr;             // BP_LINEAR_X64: segment totals, per workgroup (in d_packed)
     struct PackRange { int first, count, kind, rows; };
     std::vector<PackRange> pack_ranges;  // one per group: jobs of one kind
     void* d_fft_work = nullptr;          // two-pass transforms (n > 16384): work rows
@@ -152,7 +152,6 @@ void plan_free(rv_plan_t p)
     (void)hipFree(p->d_gscale);
     (void)hipFree(p->d_tgeom);
     (void)hipFree(p->d_pack_jobs);
-    (void)hipFree(p->d_xsum);
     (void)hipFree(p->d_fft_work);
     delete p;
 }
@@ -713,10 +712,23 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
                 n_half += is_x(G.mode) ? 2 * (size_t)rv::bp_slices_per_item(G.mode)
                                               : G.mode != rv::BP_LINEAR2 && G.mode != rv::BP_LINEAR4;
             }
+    // segment totals of the 64-slice items, behind the packed rows: an allocation of their own
+    // (64 MiB) costs a plan 0.4 ms more to make and free
+    size_t x_items = 0;
+    for (const auto& G : p->groups)
+        if (is_x(G.mode)) {
+            size_t n = 0;
+            for (int s : G.slices) n += (size_t)p->sl[s].tiles_x * p->sl[s].tiles_y;
+            x_items = std::max(x_items, n);
+        }
+    const size_t x_wgs = std::min(x_items, (size_t)rv::device_cu_count(device));
+    const size_t xsum_off = packed_bytes;
+    packed_bytes += sizeof(float) * rv::kBpxPart * x_wgs;
     std::vector<rv::PackJob> pack_jobs;
     if (packed_bytes &&
         !rv::hip_ok(hipMalloc(&p->d_packed, packed_bytes), "packed multi-slice rows"))
         return fail(p, std::string("plan allocation failed: ") + RecviewLastMessage());
+    if (x_wgs) p->d_xsum = (float*)(p->d_packed + xsum_off);
     if (n_half && !rv::hip_ok(hipMalloc(&p->d_gscale, sizeof(float) * n_half), "item scales"))
         return fail(p, std::string("plan allocation failed: ") + RecviewLastMessage());
     size_t packed_off = 0, half_idx = 0;
@@ -777,7 +789,6 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
             return fail(p, std::string("plan set-up failed: ") + RecviewLastMessage());
     }
 
-    int x_grid = 0;
     for (auto& G : p->groups) {
         // slice order inside the group: longest projection lists first
         std::vector<int> ord = G.slices;
@@ -886,8 +897,7 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
             return fail(p, std::string("plan upload failed: ") + RecviewLastMessage());
         if (is_x(G.mode)) {
             rv::bpx_prepare();
-            G.grid = std::min(rv::device_cu_count(device), G.total_items);     // one workgroup per CU
-            x_grid = std::max(x_grid, G.grid);
+            G.grid = std::min((int)x_wgs, G.total_items);                      // one workgroup per CU
             if (!rv::hip_ok(hipMalloc(&G.d_rest, sizeof(rv::BpSlice) * G.rest.size()), "slice table") ||
                 !rv::hip_ok(hipMalloc(&G.d_rest_order, sizeof(int) * G.rest_items), "work list") ||
                 !rv::hip_ok(hipMemcpy(G.d_rest, G.rest.data(), sizeof(rv::BpSlice) * G.rest.size(),
@@ -908,10 +918,6 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
         }
     }
     p->cur_out.assign(nslices, nullptr);
-    if (!xg_tab.empty()) {
-        if (!rv::hip_ok(hipMalloc(&p->d_xsum, sizeof(float) * rv::kBpxPart * x_grid), "segment totals"))
-            return fail(p, std::string("plan allocation failed: ") + RecviewLastMessage());
-    }
     if (!pack_jobs.empty()) {
         p->n_pack = (int)pack_jobs.size();
         if (!rv::hip_ok(hipMalloc(&p->d_pack_jobs, sizeof(rv::PackJob) * pack_jobs.size()), "pack jobs") ||
