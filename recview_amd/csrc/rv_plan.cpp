@@ -187,7 +187,7 @@ bool upload_slices(rv_plan_t p, void* const* d_out, hipStream_t st, bool all)
                 G.h[q].out = d_out[s];
                 add(&G.d_slices[q].out, d_out[s]);
             }
-            for (int e = 0; e + 1 < rv::BP_MAX_SLICES_PER_ITEM; e++) {
+            for (int e = 0; e + 1 < rv::bp_slices_per_item(G.mode); e++) {
                 const int s2 = G.others[q][e];
                 if (s2 >= 0 && (all || p->cur_out[s2] != d_out[s2])) {
                     G.h[q].out_x[e] = d_out[s2];
