@@ -215,11 +215,29 @@ __global__ void __launch_bounds__(256) bp_sub_kernel(BpLaunch L, SubTile E)
 // tiles (64 x 128 and 128 x 64 below 700^2) / parts: 384^2 x 225 270 / 52, 512^2 x 450 505 / 91,
 // 600^2 x 450 506 / 109, 1024^2 x 900 562 / 268, 1400^2 x 1200 (484) 767 / 642.
 // (Tiles counted as 64 x 64 pixels, whatever the tile configuration.)
-int bp_sub_parts(int mode, int tile, int total_items)
+// Whole tiles come sooner where they fill the chip sooner or cost less to stage: 32 x 32
+// and 32 x 64 tiles, which are two to four times as many (four slices of 1200^2 x 900 on
+// 32 x 32: 500 whole, 764 in parts; pairs of 1400^2 x 900 on 32 x 64: 408 / 479; one slice of
+// 1600^2 x 900 on 32 x 64: 399 / 429); 16-bit rows, which parts convert once each (1600^2 x
+// 900: 490 / 515; 1400^2 x 900: 430 / 426); and, when a launch takes no work from a queue
+// (which costs it a launch of its own and an atomic per tile), pairs and fours of few
+// angles (1400^2 x 8, pairs: 26 / 30, from a queue 36 / 30) and fours of many tiles (1400^2 x
+// 65: 86 / 90).  Over 1992 shapes, modes and tiles parts were chosen for nothing that they
+// make more than 3% slower, and on average gained 1.53.
+int bp_sub_parts(int mode, int tile, int total_items, int nang, bool rows16, bool queue)
 {
     const long long n = (long long)total_items * bp_tile_side(tile) * bp_tile_h(tile) / 4096;
-    if (mode == BP_LINEAR) return n <= 48 ? 16 : n <= 96 ? 8 : n <= 640 ? 4 : 0;
-    if (mode == BP_LINEAR2 || mode == BP_LINEAR4) return n <= 80 ? 16 : n <= 150 ? 8 : n <= 512 ? 4 : 0;
+    const bool small = tile == 2 || tile == 4, few = nang < 32;
+    if (mode == BP_LINEAR) {
+        int most = rows16 && (tile == 0 || small) ? 512 : 640;
+        if (small && !few) most = queue && !rows16 ? 512 : 256;
+        return n <= 48 ? 16 : n <= 96 ? 8 : n <= most ? 4 : 0;
+    }
+    if (mode == BP_LINEAR2 || mode == BP_LINEAR4) {
+        if (n > 512 || (small && total_items > 512 && !(few && queue))) return 0;
+        if (tile == 0 && !queue && ((few && n > 150) || (mode == BP_LINEAR4 && n > 400))) return 0;
+        return n <= 80 ? 16 : n <= 150 ? 8 : 4;
+    }
     return 0;
 }
 

@@ -752,7 +752,10 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
             base += p->sl[s].tiles_x * p->sl[s].tiles_y;
         }
         G.total_items = base;
-        if (!is_x(G.mode)) G.parts = rv::bp_sub_parts(G.mode, G.tile, G.total_items);
+        int nang = 0;
+        for (int s : G.slices) nang = std::max(nang, p->sl[s].nang);
+        if (!is_x(G.mode))
+            G.parts = rv::bp_sub_parts(G.mode, G.tile, G.total_items, nang, p->store != 0, opt->persistent != 0);
         if (!tg_allowed || G.parts || !rv::bp_has_tgeom(G.mode)) continue;
         G.tgeom = true;
         for (int s : G.slices) {
