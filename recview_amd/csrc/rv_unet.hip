@@ -703,18 +703,22 @@ hipError_t launch_conv3x3_wgrad(const WgradArgs& a, hipStream_t s) {
 }
 
 // Column sums of part[nsplit][n] into out and, in the last blocks, of part2[nsplit][n2]
-// into out2.  Block: 64 columns (256-byte rows), wave w takes splits w, w + 16, ...,
-// eight loads in flight, and the waves' sums meet in LDS.  Bound by reading the parts:
-// one thread per column had too few waves (n = 9216, 1024 splits: 36 blocks) and a serial
-// chain of loads, 3.2 ms of the 14.0 ms of a 16 x 512^2 gradient; that now takes 10.9 ms.
-constexpr int SUM_WAVES = 16;
-__global__ __launch_bounds__(64 * SUM_WAVES) void sum_splits_kernel(const float* part, int nsplit, int n, float* out,
-                                                                    const float* part2, int n2, float* out2) {
-    __shared__ float red[SUM_WAVES][64];
-    const int l = threadIdx.x & 63, w = threadIdx.x >> 6, nb = (n + 63) / 64;
-    int i = blockIdx.x * 64 + l;
+// into out2.  WAVES waves share 64 columns (256-byte rows), wave w taking the splits w, w +
+// WAVES, ..., eight loads in flight, and their sums meet in LDS; a workgroup holds GROUPS
+// such columns.  Bound by reading the parts: one thread per column had too few waves
+// (n = 9216, 1024 splits: 36 blocks) and a serial chain of loads, 3.2 ms of the 14.0 ms of
+// a 16 x 512^2 gradient; that now takes 10.9 ms.
+template <int WAVES, int GROUPS>
+__global__ __launch_bounds__(64 * WAVES * GROUPS) void sum_splits_kernel(const float* part, int nsplit, int n,
+                                                                         float* out, const float* part2, int n2,
+                                                                         float* out2) {
+    constexpr int COLS = 64 * GROUPS;
+    __shared__ float red[WAVES][COLS];
+    const int wave = threadIdx.x >> 6, w = wave % WAVES, c = (wave / WAVES) * 64 + (threadIdx.x & 63);
+    const int nb = (n + COLS - 1) / COLS;
+    int i = blockIdx.x * COLS + c;
     if (blockIdx.x >= nb) {
-        i -= nb * 64;
+        i -= nb * COLS;
         part = part2;
         n = n2;
         out = out2;
@@ -723,27 +727,44 @@ __global__ __launch_bounds__(64 * SUM_WAVES) void sum_splits_kernel(const float*
     if (i < n) {
         const float* p = part + i;
         int k = w;
-        for (; k + 7 * SUM_WAVES < nsplit; k += 8 * SUM_WAVES) {
+        for (; k + 7 * WAVES < nsplit; k += 8 * WAVES) {
             float v[8];
 #pragma unroll
-            for (int e = 0; e < 8; e++) v[e] = p[(long long)(k + e * SUM_WAVES) * n];
+            for (int e = 0; e < 8; e++) v[e] = p[(long long)(k + e * WAVES) * n];
             s += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
         }
-        for (; k < nsplit; k += SUM_WAVES) s += p[(long long)k * n];
+        for (; k < nsplit; k += WAVES) s += p[(long long)k * n];
     }
-    red[w][l] = s;
-    __syncthreads();
-    if (w == 0 && i < n) {
+    if constexpr (WAVES > 1) {
+        red[w][c] = s;
+        __syncthreads();
+        if (w == 0 && i < n) {
 #pragma unroll
-        for (int k = 1; k < SUM_WAVES; k++) s += red[k][l];
+            for (int k = 1; k < WAVES; k++) s += red[k][c];
+            out[i] = s;
+        }
+    } else if (i < n) {
         out[i] = s;
     }
 }
 
+template <int WAVES, int GROUPS>
+static void sum_splits(const float* part, int nsplit, int n, float* out, hipStream_t s, const float* part2, int n2,
+                       float* out2) {
+    constexpr int COLS = 64 * GROUPS;
+    hipLaunchKernelGGL((sum_splits_kernel<WAVES, GROUPS>), dim3((n + COLS - 1) / COLS + (n2 + COLS - 1) / COLS),
+                       dim3(64 * WAVES * GROUPS), 0, s, part, nsplit, n, out, part2, n2, out2);
+}
+
 hipError_t launch_sum_splits(const float* part, int nsplit, int n, float* out, hipStream_t s, const float* part2,
                              int n2, float* out2) {
-    hipLaunchKernelGGL(sum_splits_kernel, dim3((n + 63) / 64 + (n2 + 63) / 64), dim3(64 * SUM_WAVES), 0, s, part,
-                       nsplit, n, out, part2, n2, out2);
+    // as many waves as the chip needs: with sixteen for 64 columns of a wide layer, which has
+    // few parts, most found nothing to add (whole weight gradient, 16 / 4 / 1 waves, us: 1179648
+    // columns of 4 parts 96 / 75 / 73, 589824 of 16 87 / 79 / 73, 147456 of 16 65 / 64 / 62;
+    // 9216 of 1024 75 / 82 / 115)
+    if (n >= 1 << 18) sum_splits<1, 4>(part, nsplit, n, out, s, part2, n2, out2);
+    else if (n >= 1 << 16) sum_splits<4, 1>(part, nsplit, n, out, s, part2, n2, out2);
+    else sum_splits<16, 1>(part, nsplit, n, out, s, part2, n2, out2);
     return hipGetLastError();
 }
 

@@ -303,3 +303,20 @@ def test_edge_layer_gradients_of_an_infinite_target(W):
     taps = np.isfinite(g[w:w + 9 * ci].reshape(3, 3, ci))
     assert taps[:, 2].all()                            # the neighbour to the right is outside
     assert not taps[:, :2].all()
+
+
+@pytest.mark.parametrize("cin,cout,B,H,W", [
+    (128, 128, 1, 8, 16), (128, 64, 1, 17, 33), (128, 128, 2, 40, 70),    # four waves share a column's parts
+    (256, 128, 1, 8, 8), (512, 256, 1, 9, 40), (256, 128, 3, 70, 90)])    # one does
+def test_conv_weight_gradient_sums_of_wide_layers(cin, cout, B, H, W):
+    """The sums of a wide layer's weight-gradient parts, from one part to as many as the
+    layer takes, against the FP64 oracle (FP32 sums of at most 18900 products: well below
+    sqrt(18900) / 2 * 2^-24 = 4.1e-6 of the result's RMS)."""
+    rng = np.random.default_rng(cin + cout + H)
+    g = U.bf16_round(rng.standard_normal((B, H, W, cout)))
+    x = U.bf16_round(rng.standard_normal((B, H, W, cin)))
+    dw, db = RU.conv3x3_wgrad(bf(g), bf(x), cin, cout, (B, H, W))
+    torch.cuda.synchronize()
+    rw, rb = U.conv3x3_wgrad(g, x)
+    assert rel(dw.double().cpu().numpy(), rw) < 1e-5
+    assert rel(db.double().cpu().numpy(), rb) < 1e-5
