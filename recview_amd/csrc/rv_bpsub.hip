@@ -215,27 +215,37 @@ __global__ void __launch_bounds__(256) bp_sub_kernel(BpLaunch L, SubTile E)
 // tiles (64 x 128 and 128 x 64 below 700^2) / parts: 384^2 x 225 270 / 52, 512^2 x 450 505 / 91,
 // 600^2 x 450 506 / 109, 1024^2 x 900 562 / 268, 1400^2 x 1200 (484) 767 / 642.
 // (Tiles counted as 64 x 64 pixels, whatever the tile configuration.)
-// Whole tiles come sooner where they fill the chip sooner or cost less to stage: 32 x 32
-// and 32 x 64 tiles, which are two to four times as many (four slices of 1200^2 x 900 on
-// 32 x 32: 500 whole, 764 in parts; pairs of 1400^2 x 900 on 32 x 64: 408 / 479; one slice of
-// 1600^2 x 900 on 32 x 64: 399 / 429); 16-bit rows, which parts convert once each (1600^2 x
-// 900: 490 / 515; 1400^2 x 900: 430 / 426); and, when a launch takes no work from a queue
-// (which costs it a launch of its own and an atomic per tile), pairs and fours of few
-// angles (1400^2 x 8, pairs: 26 / 30, from a queue 36 / 30) and fours of many tiles (1400^2 x
-// 65: 86 / 90).  Over 1992 shapes, modes and tiles parts were chosen for nothing that they
-// make more than 3% slower, and on average gained 1.53.
-int bp_sub_parts(int mode, int tile, int total_items, int nang, bool rows16, bool queue)
+// Parts of 32 x 32 pixels fill the chip once with 256 tiles and twice with 512.  Whole tiles
+// come sooner where they fill it sooner or cost less to stage: 32 x 32 and 32 x 64 tiles,
+// which are two to four times as many (whole / parts, us: four slices of 1200^2 x 900 on 32 x
+// 32 500 / 764, pairs of 1400^2 x 900 on 32 x 64 408 / 479, one slice of 1600^2 x 900 there 399 /
+// 429), and 16-bit rows, whose samples cost more to stage (1600^2 x 900 493 / 525).  They come
+// later when a launch takes its tiles from a queue and its angles are few, since it then
+// mostly takes tiles (an atomic each, and a launch that clears the counter: pairs of 1376^2 x 24
+// on 32 x 32 63 / 34), and pairs with chunks shorter than the default (1100^2 x 700 on 32 x 64
+// in chunks of 12: 353 / 287); without a queue, pairs and fours of few angles are whole
+// (1400^2 x 1 26 / 31).  Lone 32 x 32 tiles sit six to a CU, so that from 1536 on a second
+// round begins (1280^2 x 1500 641 / 495).  Of 3986 measured launches the rule makes one more
+// than 5% slower than whole tiles.
+int bp_sub_parts(int mode, int tile, int chunk, int total_items, int nang, bool rows16, bool queue)
 {
     const long long n = (long long)total_items * bp_tile_side(tile) * bp_tile_h(tile) / 4096;
-    const bool small = tile == 2 || tile == 4, few = nang < 32;
+    const bool small = tile == 2 || tile == 4;
     if (mode == BP_LINEAR) {
-        int most = rows16 && (tile == 0 || small) ? 512 : 640;
-        if (small && !few) most = queue && !rows16 ? 512 : 256;
+        const bool brief = nang < (queue ? 100 : 32);
+        int most = 640;
+        if (tile == 4 && !brief) most = queue ? (rows16 ? 430 : 512) : rows16 ? 256 : 430;
+        else if (tile == 2 && !brief && !(queue && !rows16)) most = n > 384 ? 512 : 256;
+        else if ((tile == 0 || small) && rows16 && !(brief && queue)) most = 512;
         return n <= 48 ? 16 : n <= 96 ? 8 : n <= most ? 4 : 0;
     }
     if (mode == BP_LINEAR2 || mode == BP_LINEAR4) {
-        if (n > 512 || (small && total_items > 512 && !(few && queue))) return 0;
-        if (tile == 0 && !queue && ((few && n > 150) || (mode == BP_LINEAR4 && n > 400))) return 0;
+        const bool pair = mode == BP_LINEAR2;
+        int most = 512;
+        const bool late = (queue && nang < (pair ? 100 : 32)) || (pair && chunk < bp_default_chunk(mode, tile));
+        if (small && !late) most = tile == 4 || (pair && queue) ? 256 : 128;
+        if (n > most) return 0;
+        if (tile == 0 && !queue && ((n > 150 && nang < 8) || (n > 256 && nang < (pair ? 20 : 100)))) return 0;
         return n <= 80 ? 16 : n <= 150 ? 8 : 4;
     }
     return 0;

@@ -755,7 +755,8 @@ int rvPlanCreate(rv_plan_t* out, int device, const RvSliceSpec* specs, int nslic
         int nang = 0;
         for (int s : G.slices) nang = std::max(nang, p->sl[s].nang);
         if (!is_x(G.mode))
-            G.parts = rv::bp_sub_parts(G.mode, G.tile, G.total_items, nang, p->store != 0, opt->persistent != 0);
+            G.parts = rv::bp_sub_parts(G.mode, G.tile, G.chunk, G.total_items, nang, p->store != 0,
+                                       opt->persistent != 0);
         if (!tg_allowed || G.parts || !rv::bp_has_tgeom(G.mode)) continue;
         G.tgeom = true;
         for (int s : G.slices) {
