@@ -149,31 +149,27 @@ __global__ void __launch_bounds__(256) bp_sub_kernel(BpLaunch L, SubTile E)
             fetch_rows(a0 + CH);
             fetch_entry(a0 + 2 * CH);
         }
-        // angles in fours; those past the last, up to three, add zeros
-        const int na = min(CH, nang - a0);
-        for (int a4 = 0; a4 < na; a4 += 4) {
+#pragma unroll 4
+        for (int a = 0; a < CH; a++) {                 // angles past the last add zeros
+            const float4 tb = tab[a];
+            const T* seg = data + __float_as_int(tb.w);
+            const float base = fmaf(dyl, tb.y, fmaf(dxl, tb.x, tb.z));
 #pragma unroll
-            for (int a = a4; a < a4 + 4; a++) {
-                const float4 tb = tab[a];
-                const T* seg = data + __float_as_int(tb.w);
-                const float base = fmaf(dyl, tb.y, fmaf(dxl, tb.x, tb.z));
+            for (int j = 0; j < PY; j++) {
+                const float bj = fmaf(yj + 8 * j, tb.y, base);
 #pragma unroll
-                for (int j = 0; j < PY; j++) {
-                    const float bj = fmaf(yj + 8 * j, tb.y, base);
+                for (int i = 0; i < PX; i++) {
+                    const float u = fmaf(xi + 8 * i, tb.x, bj);
+                    const T* p = seg + (int)u;
+                    if constexpr (NS == 1) {
+                        const float2 v = p[0];
+                        acc[0][j][i] += fmaf(u, v.y, v.x);
+                    } else {
 #pragma unroll
-                    for (int i = 0; i < PX; i++) {
-                        const float u = fmaf(xi + 8 * i, tb.x, bj);
-                        const T* p = seg + (int)u;
-                        if constexpr (NS == 1) {
-                            const float2 v = p[0];
-                            acc[0][j][i] += fmaf(u, v.y, v.x);
-                        } else {
-#pragma unroll
-                            for (int q = 0; q < NQ; q++) {
-                                const float4 v = p[q * SEG];
-                                acc[2 * q][j][i] += fmaf(u, v.y, v.x);
-                                acc[2 * q + 1][j][i] += fmaf(u, v.w, v.z);
-                            }
+                        for (int q = 0; q < NQ; q++) {
+                            const float4 v = p[q * SEG];
+                            acc[2 * q][j][i] += fmaf(u, v.y, v.x);
+                            acc[2 * q + 1][j][i] += fmaf(u, v.w, v.z);
                         }
                     }
                 }
