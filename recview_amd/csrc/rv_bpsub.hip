@@ -211,40 +211,62 @@ __global__ void __launch_bounds__(256) bp_sub_kernel(BpLaunch L, SubTile E)
 // tiles (64 x 128 and 128 x 64 below 700^2) / parts: 384^2 x 225 270 / 52, 512^2 x 450 505 / 91,
 // 600^2 x 450 506 / 109, 1024^2 x 900 562 / 268, 1400^2 x 1200 (484) 767 / 642.
 // (Tiles counted as 64 x 64 pixels, whatever the tile configuration.)
-// Parts of 32 x 32 pixels fill the chip once with 256 tiles and twice with 512.  Whole tiles
-// come sooner where they fill it sooner or cost less to stage: 32 x 32 and 32 x 64 tiles,
-// which are two to four times as many (whole / parts, us: four slices of 1200^2 x 900 on 32 x
-// 32 500 / 764, pairs of 1400^2 x 900 on 32 x 64 408 / 479, one slice of 1600^2 x 900 there 399 /
-// 429), and 16-bit rows, whose samples cost more to stage (1600^2 x 900 493 / 525).  They come
-// later when a launch takes its tiles from a queue and its angles are few, since it then
-// mostly takes tiles (an atomic each, and a launch that clears the counter: pairs of 1376^2 x 24
-// on 32 x 32 63 / 34), and pairs with chunks shorter than the default (1100^2 x 700 on 32 x 64
-// in chunks of 12: 353 / 287); without a queue, pairs and fours of few angles are whole
-// (1400^2 x 1 26 / 31).  Lone 32 x 32 tiles sit six to a CU, so that from 1536 on a second
-// round begins (1280^2 x 1500 641 / 495).  Of 3986 measured launches the rule makes one more
-// than 5% slower than whole tiles.
+// Where whole tiles take over depends on what each side costs.  Parts of 32 x 32 pixels fill
+// the chip once with 256 tiles and twice with 512, and sum whole chunks of 16 angles in
+// pairs and fours (1400^2 x 20, fours: 50 whole, 60 in parts).  32 x 32 and 32 x 64 tiles are
+// two to four times as many, so that whole they fill it sooner (four slices of 1200^2 x 900
+// on 32 x 32: 500 / 764, pairs of 1400^2 x 900 on 32 x 64 408 / 479); lone ones sit six to a CU,
+// a second round beginning with 1536 of them (1280^2 x 1500 641 / 495).  16-bit rows cost
+// parts more to stage (1600^2 x 900 493 / 525); chunks below the default cost whole pairs more
+// (1100^2 x 700 on 32 x 64 in chunks of 12: 353 / 287).  A queue costs whole tiles an atomic each and a
+// launch that clears its counter, which is most of their time when angles are few (pairs of
+// 1376^2 x 24 on 32 x 32: 63 / 34, without a queue 33 / 34).  The lines below were read off
+// 6960 measured launches; they make none more than 5% slower than whole tiles.
+static int bp_sub_most(int mode, int tile, int chunk, long long n, int nang, bool rows16, bool queue)
+{
+    const int round = n > 384 ? 512 : 256;                 // small tiles: gains up to here, and again from 384 on
+    if (mode == BP_LINEAR) {
+        if (tile == 2) {
+            if (queue) return nang < 200 || !rows16 ? 640 : round;
+            return nang >= 32 ? round : rows16 ? 512 : 640;
+        }
+        if (tile == 4) {
+            if (queue) return nang < 200 ? 640 : rows16 ? 430 : 512;
+            return rows16 || nang < 32 ? 256 : 430;
+        }
+        if (tile == 0 && rows16) return queue && nang < 100 ? 640 : nang < 64 ? 440 : 512;
+        return queue || nang >= 32 ? 640 : 570;
+    }
+    if (mode == BP_LINEAR2) {
+        if (tile == 2 || tile == 4) {
+            if (queue) return nang < 200 || chunk < bp_default_chunk(mode, tile) ? 512 : 256;
+            return tile == 4 ? (nang < 32 ? 128 : 256) : nang < 100 ? 80 : 128;
+        }
+        if (tile == 0 && !queue)                            // 380: over a fifth more angles summed than there are
+            return nang < 8 ? 150 : nang < 20 ? 256 : 5 * (-nang & 15) > nang ? 380 : 512;
+        return 512;
+    }
+    if (mode == BP_LINEAR4) {
+        if (tile == 2) {
+            if (queue) return nang < 32 ? 512 : nang < 100 ? round : 128;
+            return nang < 40 ? 80 : 128;
+        }
+        if (tile == 4) return queue ? (nang < 16 ? 512 : 256) : nang < 40 ? 80 : 256;
+        if (tile == 0) {
+            if (queue) return nang < 36 ? 256 : 512;
+            return nang < 8 ? 100 : nang < 100 ? 256 : nang < 200 ? 400 : 512;
+        }
+        return !queue && nang < 8 ? 256 : 512;
+    }
+    return 0;
+}
+
 int bp_sub_parts(int mode, int tile, int chunk, int total_items, int nang, bool rows16, bool queue)
 {
     const long long n = (long long)total_items * bp_tile_side(tile) * bp_tile_h(tile) / 4096;
-    const bool small = tile == 2 || tile == 4;
-    if (mode == BP_LINEAR) {
-        const bool brief = nang < (queue ? 100 : 32);
-        int most = 640;
-        if (tile == 4 && !brief) most = queue ? (rows16 ? 430 : 512) : rows16 ? 256 : 430;
-        else if (tile == 2 && !brief && !(queue && !rows16)) most = n > 384 ? 512 : 256;
-        else if ((tile == 0 || small) && rows16 && !(brief && queue)) most = 512;
-        return n <= 48 ? 16 : n <= 96 ? 8 : n <= most ? 4 : 0;
-    }
-    if (mode == BP_LINEAR2 || mode == BP_LINEAR4) {
-        const bool pair = mode == BP_LINEAR2;
-        int most = 512;
-        const bool late = (queue && nang < (pair ? 100 : 32)) || (pair && chunk < bp_default_chunk(mode, tile));
-        if (small && !late) most = tile == 4 || (pair && queue) ? 256 : 128;
-        if (n > most) return 0;
-        if (tile == 0 && !queue && ((n > 150 && nang < 8) || (n > 256 && nang < (pair ? 20 : 100)))) return 0;
-        return n <= 80 ? 16 : n <= 150 ? 8 : 4;
-    }
-    return 0;
+    if (n > bp_sub_most(mode, tile, chunk, n, nang, rows16, queue)) return 0;
+    if (mode == BP_LINEAR) return n <= 48 ? 16 : n <= 96 ? 8 : 4;
+    return n <= 80 ? 16 : n <= (tile == 2 ? 128 : 150) ? 8 : 4;
 }
 
 template <int NS, int PX, int PY>

@@ -217,8 +217,8 @@ inline int work_run(int total_items, bool deal)
 
 void launch_bp(const BpLaunch& L, int grid, hipStream_t stream);
 // Workgroups that share 64 x 64 pixels of a tile (launch_bp_sub), for launches of one FP32
-// slice, pair or four per item whose tiles are too few; 0: whole tiles.  nang: the largest
-// angle count; rows16: 16-bit filtered rows; queue: a persistent launch.
+// slice, pair or four per item whose tiles are too few; 0: whole tiles.  chunk: of whole
+// tiles; nang: the largest angle count; rows16: 16-bit filtered rows; queue: a persistent launch.
 int bp_sub_parts(int mode, int tile, int chunk, int total_items, int nang, bool rows16, bool queue);
 void launch_bp_sub(const BpLaunch& L, int parts, hipStream_t stream);
 
