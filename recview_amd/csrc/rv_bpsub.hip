@@ -216,7 +216,7 @@ __global__ void __launch_bounds__(256) bp_sub_kernel(BpLaunch L, SubTile E)
 // pairs and fours (1400^2 x 20, fours: 50 whole, 60 in parts).  32 x 32 and 32 x 64 tiles are
 // two to four times as many, so that whole they fill it sooner (four slices of 1200^2 x 900
 // on 32 x 32: 500 / 764, pairs of 1400^2 x 900 on 32 x 64 408 / 479); lone ones sit six to a CU,
-// a second round beginning with 1536 of them (1280^2 x 1500 641 / 495).  16-bit rows cost
+// a second set beginning with 1536 of them (1280^2 x 1500 641 / 495).  16-bit rows cost
 // parts more to stage (1600^2 x 900 493 / 525); chunks below the default cost whole pairs more
 // (1100^2 x 700 on 32 x 64 in chunks of 12: 353 / 287).  A queue costs whole tiles an atomic each and a
 // launch that clears its counter, which is most of their time when angles are few (pairs of
@@ -224,11 +224,11 @@ __global__ void __launch_bounds__(256) bp_sub_kernel(BpLaunch L, SubTile E)
 // 6960 measured launches; they make none more than 5% slower than whole tiles.
 static int bp_sub_most(int mode, int tile, int chunk, long long n, int nang, bool rows16, bool queue)
 {
-    const int round = n > 384 ? 512 : 256;                 // small tiles: gains up to here, and again from 384 on
+    const int filled = n > 384 ? 512 : 256;                 // small tiles: gains up to here, and again from 384 on
     if (mode == BP_LINEAR) {
         if (tile == 2) {
-            if (queue) return nang < 200 || !rows16 ? 640 : round;
-            return nang >= 32 ? round : rows16 ? 512 : 640;
+            if (queue) return nang < 200 || !rows16 ? 640 : filled;
+            return nang >= 32 ? filled : rows16 ? 512 : 640;
         }
         if (tile == 4) {
             if (queue) return nang < 200 ? 640 : rows16 ? 430 : 512;
@@ -248,7 +248,7 @@ static int bp_sub_most(int mode, int tile, int chunk, long long n, int nang, boo
     }
     if (mode == BP_LINEAR4) {
         if (tile == 2) {
-            if (queue) return nang < 32 ? 512 : nang < 100 ? round : 128;
+            if (queue) return nang < 32 ? 512 : nang < 100 ? filled : 128;
             return nang < 40 ? 80 : 128;
         }
         if (tile == 4) return queue ? (nang < 16 ? 512 : 256) : nang < 40 ? 80 : 256;
